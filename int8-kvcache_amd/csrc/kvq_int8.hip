@@ -638,13 +638,22 @@ __device__ __forceinline__ long long lane_value64(long long x, int l) {
   return (long long)(((unsigned long long)hi << 32) | lo);
 }
 
-// The plan (total units, chunk) and the request holding unit pos0 = worker * chunk -- its index, the
-// unit its segments start at and its work -- in two scans over the requests (their work is read once;
-// up to PLAN_CACHE * 64 requests stay in registers). Every workgroup computes the same plan at once
+// The plan (total units, chunk), the worker this workgroup is (below) and the request holding unit pos0 =
+// worker * chunk -- its index, the unit its segments start at and its work -- in two scans over the
+// requests (their work is read once; up to PLAN_CACHE * 64 requests stay in registers). Every workgroup computes the same plan at once
 // from the same few lines of cu_seqlens_q / seq_lens, so the scans run on DPP rather than through LDS
 // permutes (the plan took ~7 us of a 62 us verification batch with 64-bit shuffle reductions).
 constexpr int PLAN_CACHE = 4;
-__device__ Plan plan_and_locate(const AttnArgs& a, int worker, int lane, int& r_out, long long& start_out,
+// The worker a workgroup is follows from the plan too: workgroups are dispatched round-robin over
+// the XCDs, and XCD x takes a contiguous range of the workers that hold units (so one XCD's L2 sees whole
+// requests' block-table rows and q): the blocks b = x (mod 8), active / 8 of them or one more, take the
+// workers [x q + min(x, rem), ...) for active = 8 q + rem -- consecutive ranges that tile [0, active)
+// exactly. Counting the workers with units, not the grid, spreads a small batch over all 8 XCDs: an XCD
+// draws about an eighth of the HBM bandwidth, and a batch with fewer pieces than workgroups otherwise
+// filled the first XCDs only (attention + merge in a graph, same box: 1 x 4,096 keys 18.2 -> 15.0 us,
+// 8 requests of about 2k 21.9 -> 18.1, 1 x 32k 48.8 -> 36.7, 4 x 8-token verification of 4k 24.5 -> 20.3;
+// full grids unchanged). KVQ_XCD_ORDER=0 makes worker = block.
+__device__ Plan plan_and_locate(const AttnArgs& a, int lane, int& worker_out, int& r_out, long long& start_out,
                                 ReqWork& w_out) {
   long long u[PLAN_CACHE];
   int tk[PLAN_CACHE], ql[PLAN_CACHE], ln[PLAN_CACHE];
@@ -675,7 +684,15 @@ __device__ Plan plan_and_locate(const AttnArgs& a, int worker, int lane, int& r_
     ch = max(ch, (long long)a.min_tiles);
   }
   p.chunk = uniform64(max(ch, 1ll));
-  const long long pos = (long long)worker * p.chunk;
+  const int active = (int)min((long long)a.workers, udiv_plan(p.total + p.chunk - 1, p.chunk));
+  int worker = blockIdx.x;
+  if (a.xcd_order) {
+    const int q = active / NUM_XCDS, rem = active % NUM_XCDS;
+    const int wx = blockIdx.x % NUM_XCDS, wi = blockIdx.x / NUM_XCDS;
+    worker = wi < q + (wx < rem ? 1 : 0) ? wx * q + min(wx, rem) + wi : active;
+  }
+  worker_out = worker;
+  const long long pos = worker < active ? (long long)worker * p.chunk : p.total;
   long long base = 0;
   r_out = a.num_seqs;
   start_out = p.total;
@@ -1353,21 +1370,10 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
   const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int rtile = wave % a.rt, kspl = wave / a.rt;  // row tile and key split of this wavefront
   extern __shared__ float merge_lds[];  // (ksplit - 1) * rt slots, sized at launch (none without key splits)
-  // workgroups are dispatched round-robin over the XCDs: give each XCD a contiguous range of workers
-  // (so one XCD's L2 sees whole requests' block-table rows and q); KVQ_XCD_ORDER=0 turns it off.
-  // XCD x holds the blocks b = x (mod 8), q + (x < rem) of them for W = 8 q + rem, and takes the
-  // workers [x q + min(x, rem), ...) -- consecutive ranges that tile [0, W) exactly.
-  int worker = blockIdx.x;
-  {  // no branch before the plan: its argument loads go out in one batch
-    const int q = a.workers / NUM_XCDS, rem = a.workers % NUM_XCDS;
-    const int wx = blockIdx.x % NUM_XCDS, wi = blockIdx.x / NUM_XCDS;
-    worker = a.xcd_order ? wx * q + min(wx, rem) + wi : worker;
-    worker = (int)blockIdx.x < a.workers ? worker : a.workers;   // past the grid's workers: no units
-  }
-  int r;
+  int worker, r;
   long long rstart;
   ReqWork w;
-  const Plan pl = plan_and_locate(a, worker, lane, r, rstart, w);
+  const Plan pl = plan_and_locate(a, lane, worker, r, rstart, w);
   long long pos = (long long)worker * pl.chunk;
   const long long end = min(pos + pl.chunk, pl.total);
   if (pos >= end || r >= a.num_seqs) return;
@@ -1963,17 +1969,10 @@ __global__ __launch_bounds__(WAVE * 2 * KS) void verify_kernel(AttnArgs a) {
   float* vsl = reinterpret_cast<float*>(rings + v32_vscale_offset(D, PF, KS)) + rw * D;
   float* ksl = reinterpret_cast<float*>(rings + v32_vscale_offset(D, PF, KS)) + (2 + wave) * D;
   float* merge = reinterpret_cast<float*>(rings);
-  int worker = blockIdx.x;
-  {  // no branch before the plan: its argument loads go out in one batch
-    const int q = a.workers / NUM_XCDS, rem = a.workers % NUM_XCDS;
-    const int wx = blockIdx.x % NUM_XCDS, wi = blockIdx.x / NUM_XCDS;
-    worker = a.xcd_order ? wx * q + min(wx, rem) + wi : worker;
-    worker = (int)blockIdx.x < a.workers ? worker : a.workers;   // past the grid's workers: no units
-  }
-  int r;
+  int worker, r;
   long long rstart;
   ReqWork w;
-  const Plan pl = plan_and_locate(a, worker, lane, r, rstart, w);
+  const Plan pl = plan_and_locate(a, lane, worker, r, rstart, w);
   long long pos = (long long)worker * pl.chunk;
   const long long end = min(pos + pl.chunk, pl.total);
   if (pos >= end || r >= a.num_seqs) return;

@@ -1,0 +1,37 @@
+"""Batches that leave the chip idle: fewer pieces of work than workgroups (attn_kernel, verify_kernel)."""
+import pytest
+import torch
+from conftest import nan_like, nan_segm
+
+from kvq import cuda_kernels as ck
+from kvq import synth
+from test_gpu_kernels import check_attention, dev, int8_cache, oracle_attention
+
+pytestmark = pytest.mark.gpu
+
+# key counts of the requests: from one piece of one request up to several pieces per XCD, with counts around
+# multiples of the 8 XCDs (2 kv heads, pieces of at least 8 tiles of 32 keys)
+BATCHES = {"one_tile": [1], "one_piece": [200], "three": [200, 40, 1], "eight": [256, 256, 256, 250],
+           "nine": [300, 600, 33, 513], "long": [5000], "long_and_short": [7, 9000, 16, 1025]}
+
+
+@pytest.mark.parametrize("batch", list(BATCHES))
+@pytest.mark.parametrize("q_len", [1, 3, 8])
+def test_workgroup_order_of_small_batches(batch, q_len, monkeypatch):
+    """The XCD-aware order hands the workers that hold units to the workgroups of all 8 XCDs; every worker must
+    run exactly once, so the output equals the plain order's (worker = block) bit for bit."""
+    lens = [max(n, q_len) for n in BATCHES[batch]]
+    params = synth.channel_params(2, 128)
+    c = synth.paged_case(14, 2, [q_len] * len(lens), lens, seed=40 + q_len, params=params)
+    c["static"] = synth.calibration_scales(2, 128, params)
+    c["scale"] = 128 ** -0.5
+    kq, vq = int8_cache(c)
+    d = dev(c)
+    outs = []
+    for order in ("1", "0"):
+        monkeypatch.setenv("KVQ_XCD_ORDER", order)
+        outs.append(ck.decode_attention(d["q"], dev(kq), dev(vq), nan_like(d["q"]), d["cu"], d["seq_lens"],
+                                        d["block_table"], c["scale"], d["static"],
+                                        segm=nan_segm(d["q"].shape[0], 14, 16, 128), max_query_len=q_len))
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    check_attention(oracle_attention(c, kq, vq), outs[0], "small_batch_order", batch=batch, q_len=q_len)

@@ -189,6 +189,40 @@ int kvq_int8_prefill_attention(const void* q, int64_t q_st, int64_t q_sh, const 
                                double softmax_scale, const float* k_scale, int64_t k_scale_cols,
                                const float* v_scale, int64_t v_scale_cols, int64_t fold_scales, void* stream);
 
+/* kvq_paged_prefill_attention / kvq_int8_prefill_attention with a split work list: several entries may share a
+ * request and first row, each reading one piece of the rows' key tiles (32 keys), so that few rows over many
+ * keys fill the chip. No counterpart in the reference. Entry i is piece (tile_piece[i] & 0xffff) of
+ * (tile_piece[i] >> 16) equal shares (1 .. kvq_prefill_max_parts()) of the tiles the lengths on the device give;
+ * an entry that is its rows' only piece writes out and ignores tile_slot. The others leave fp32 partials in slot
+ * tile_slot[i] of part_out [slots, Hkv, rows_per_tile, D] and part_ml [slots, Hkv, rows_per_tile, 2], and a second
+ * kernel merges them: merge [num_merge, 4] int32 lists (request, first row, slot of piece 0, pieces), pieces in
+ * consecutive slots; every cut (request, first row) once. merge and both buffers 16-byte aligned; the buffers are
+ * scratch of the call. tile_piece NULL: the calls above. */
+int kvq_paged_prefill_attention_ex(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sb,
+                                   int64_t k_sn, int64_t k_sh, const void* v_cache, int64_t v_sb, int64_t v_sn,
+                                   int64_t v_sh, int64_t num_blocks, int64_t block_size, int64_t num_kv_heads,
+                                   int64_t head_dim, void* out, int64_t o_st, int64_t o_sh,
+                                   const int32_t* cu_seqlens_q, const int32_t* seq_lens, const int32_t* block_table,
+                                   int64_t bt_stride, int64_t num_q_heads, const int32_t* tile_req,
+                                   const int32_t* tile_row, int64_t num_tiles, int64_t rows_per_tile,
+                                   double softmax_scale, const int32_t* tile_piece, const int32_t* tile_slot,
+                                   const int32_t* merge, int64_t num_merge, float* part_out, float* part_ml,
+                                   void* stream);
+int kvq_int8_prefill_attention_ex(const void* q, int64_t q_st, int64_t q_sh, const int8_t* k_cache, int64_t k_sb,
+                                  int64_t k_sn, int64_t k_sh, const int8_t* v_cache, int64_t v_sb, int64_t v_sn,
+                                  int64_t v_sh, int64_t num_blocks, int64_t block_size, int64_t num_kv_heads,
+                                  int64_t head_dim, void* out, int64_t o_st, int64_t o_sh,
+                                  const int32_t* cu_seqlens_q, const int32_t* seq_lens, const int32_t* block_table,
+                                  int64_t bt_stride, int64_t num_q_heads, const int32_t* tile_req,
+                                  const int32_t* tile_row, int64_t num_tiles, int64_t rows_per_tile,
+                                  double softmax_scale, const float* k_scale, int64_t k_scale_cols,
+                                  const float* v_scale, int64_t v_scale_cols, int64_t fold_scales,
+                                  const int32_t* tile_piece, const int32_t* tile_slot, const int32_t* merge,
+                                  int64_t num_merge, float* part_out, float* part_ml, void* stream);
+
+/* Most pieces a split work list may cut an entry's keys into. No counterpart in the reference. */
+int kvq_prefill_max_parts(void);
+
 /* Rows per work-list entry of kvq_paged_prefill_attention. No counterpart in the reference. */
 int kvq_prefill_rows_per_tile(void);
 

@@ -2240,8 +2240,16 @@ struct PrefillArgs {
   const int* cu_q;
   const int* seq_lens;
   const int* block_table;
-  const int* tile_req;   // workgroup x: request and first row of its 64 rows
+  const int* tile_req;   // workgroup x: request and first row of its PR_ROWS rows
   const int* tile_row;
+  // split work lists (NULL: every entry reads all of its rows' keys): entry x is piece tile_piece[x] & 0xffff of
+  // the tile_piece[x] >> 16 its rows' key tiles are cut into; where there are several, its fp32 accumulators
+  // go to slot tile_slot[x] of part_out [slots, Hkv, PR_ROWS, D], the rows' reference maxima (log2 units) and
+  // denominators to part_ml [slots, Hkv, PR_ROWS, 2], and prefill_merge_kernel finishes the rows
+  const int* tile_piece;
+  const int* tile_slot;
+  float* part_out;
+  float* part_ml;
   int64_t q_st, q_sh, o_st, o_sh, k_sb, k_sn, k_sh, v_sb, v_sn, v_sh, bt_stride;  // elements
   float sm_log2;         // softmax_scale * log2(e)
   int G, lbs, num_blocks;
@@ -2292,7 +2300,7 @@ __device__ __forceinline__ uint32_t pack_bf16x2_rne(float a, float b) {
 // code x scale) or as exact bf16 codes with the scales folded into q (K) and the output (V).
 constexpr int PR_SRC_BF16 = 0, PR_SRC_I8 = 1, PR_SRC_I8_FOLD = 2;
 
-template <int D, int SRC>
+template <int D, int SRC, bool SPLIT>
 __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
   constexpr bool I8 = SRC != PR_SRC_BF16;
   constexpr bool FOLD = SRC == PR_SRC_I8_FOLD;
@@ -2342,8 +2350,17 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
     lim[rb] = L - Q + 1 + t[rb];
   }
   const int t_last = min(Q - 1, (row0 + PR_ROWS - 1) / G);
-  const int kend = max(0, min(L, L - Q + 1 + t_last));
-  const int ntiles = (kend + PR_KEYS - 1) / PR_KEYS;
+  int kend = max(0, min(L, L - Q + 1 + t_last));
+  // the key tiles [c_lo, c_hi) of this workgroup: all of them, or one piece (an equal share: the lengths read
+  // here decide, so a work list made from upper bounds still covers exactly the keys there are)
+  int c_lo = 0, c_hi = (kend + PR_KEYS - 1) / PR_KEYS;
+  if constexpr (SPLIT) {
+    const int pp = a.tile_piece[blockIdx.x], nparts = pp >> 16;
+    const int part = pp & 0xffff, each = c_hi / nparts, rem = c_hi % nparts;
+    c_lo = part * each + min(part, rem);
+    c_hi = c_lo + each + (part < rem ? 1 : 0);
+    kend = min(kend, c_hi * PR_KEYS);
+  }
   const int wt0 = wrow0 / G;
   const int lim_lo = L - Q + 1 + wt0;  // smallest limit of the wavefront's rows
 
@@ -2412,24 +2429,32 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
   const char* vh = I8 ? (const char*)a.vc + (int64_t)kvh * a.v_sh : (const char*)(a.vc + (int64_t)kvh * a.v_sh);
   // Pages as one run: when the pages the workgroup reads are consecutive ids p_0, p_0 + 1, ... and a
   // page is bs slots (the layout dequant_pages writes), key k is slot p_0 bs + k of the head's cache:
-  // the tiles' addresses need no block-table read (checked once, by every wavefront alike).
+  // the tiles' addresses need no block-table read (checked once, by every wavefront alike; four table
+  // reads in flight per lane, over the pages of this workgroup's own tiles).
   bool linear = false;
-  int pfirst = 0;
-  if (ntiles > 0 && a.contig) {
-    const int npg = ((kend - 1) >> a.lbs) + 1;
-    pfirst = __builtin_amdgcn_readfirstlane(((const __attribute__((address_space(4))) int*)bt)[0]);
-    bool bad = pfirst < 0 || pfirst > a.num_blocks - npg;
-    for (int j = lane; j < npg && !bad; j += WAVE) bad = bt[j] != pfirst + j;
+  int pfirst = 0;   // the id page 0 of the request would have (page pg_lo's minus pg_lo: may be negative)
+  if (c_hi > c_lo && a.contig) {
+    const int pg_lo = (c_lo * PR_KEYS) >> a.lbs, pg_hi = (kend - 1) >> a.lbs;
+    pfirst = __builtin_amdgcn_readfirstlane(((const __attribute__((address_space(4))) int*)bt)[pg_lo]);
+    bool bad = pfirst < 0 || pfirst > a.num_blocks - 1 - (pg_hi - pg_lo);
+    pfirst -= pg_lo;
+    for (int j0 = pg_lo + lane; j0 <= pg_hi; j0 += 4 * WAVE) {
+      int id[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) id[u] = bt[min(j0 + u * WAVE, pg_hi)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) bad |= id[u] - pfirst != min(j0 + u * WAVE, pg_hi);
+    }
     linear = !__any(bad);
   }
-  const char* klin = kh + (uint64_t)(uint32_t)pfirst * a.kpage;
-  const char* vlin = vh + (uint64_t)(uint32_t)pfirst * a.vpage;
+  const char* klin = kh + (int64_t)pfirst * a.kpage;
+  const char* vlin = vh + (int64_t)pfirst * a.vpage;
   // tile c: keys 0..15 sit in page p0 from slot (32 c) mod bs on, keys 16..31 right after them
   // (bs >= 32) or from slot 0 of page p1 (bs == 16); rows past the last key read a valid page
   // lin_t: std::true_type = the pages are one run (no block-table read), false_type = read the
   // table, bool = decide at run time
   auto issue = [&](int c, int st, auto lin_t) {
-    c = min(c, max(ntiles - 1, 0));  // past the end: reload the last tile into the free stage
+    c = min(c, c_hi - 1);  // past the end: reload the last tile into the free stage
     const int kb0 = c * PR_KEYS, klast = max(kend - 1, 0);
     const char* kb[2];
     const char* vb[2];
@@ -2781,21 +2806,21 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
     }
   };
 
-  if (ntiles > 0) {
+  if (c_hi > c_lo) {
     // ring stages of tile c (scur) and of the tile DMA'd while c is computed (snext = stage of c - 1),
     // advanced after each tile (no division in the loop). I8: scur is tile c's bf16 stage (c % 2), s8
-    // its int8 stage (c % NS8).
+    // its int8 stage (c % NS8), tiles counted from c_lo.
     // the first tiles' DMA; I8: NS8 tiles in flight, tile 0 converted once it has landed
     auto prologue = [&]() {
       if constexpr (I8) {
 #pragma unroll
-        for (int j = 0; j < NS8; ++j) issue(j, j, linear);
+        for (int j = 0; j < NS8; ++j) issue(c_lo + j, j, linear);
         wait_vm<IPW8 * (NS8 - 1)>();
         lds_barrier();
         convert(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
       } else {
 #pragma unroll
-        for (int j = 0; j < NS - 1; ++j) issue(j, j, linear);
+        for (int j = 0; j < NS - 1; ++j) issue(c_lo + j, j, linear);
       }
     };
     prologue();
@@ -2850,7 +2875,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
         snext = snext == NS - 1 ? 0 : snext + 1;
       }
     };
-    // Fast pass: tile 0 sets each row's reference maximum (acc is still zero), later tiles only
+    // Fast pass: the first tile sets each row's reference maximum (acc is still zero), later tiles only
     // accumulate. P = 2^(s c - m) stays finite and keeps its relative precision as long as no score
     // exceeds the reference by more than 60 (log2 units). Every P is at most its lane's denominator
     // l (a sum of P >= 0), so a lane whose l ends at most 2^60 (and not NaN) saw no such score;
@@ -2858,23 +2883,23 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
     // condition, which keeps the accumulators in place in registers. The tiles below J have no key
     // past any row's limit; with the page addressing fixed per loop, their loop body is one block
     // of straight-line code.
-    const int J = min(ntiles, max(lim_lo, 0) / PR_KEYS);
+    const int J = min(c_hi, max(lim_lo, 0) / PR_KEYS);
     auto fast_pass = [&](auto lin_t) {
-      next_tile(0, lin_t, std::true_type{});
+      next_tile(c_lo, lin_t, std::true_type{});
       row_top();
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) m[rb] = __builtin_fmaxf(top[rb], -1e30f);
       softmax_pv(scur);
       advance();
-      int c = 1;
+      int c = c_lo + 1;
       if constexpr (I8) {
-        // unmasked tiles in rounds of 2, tile c in bf16 stage c % 2 (1, 0 from c = 1 on)
+        // unmasked tiles in rounds of 2, tile c in bf16 stage c % 2 (1, 0 from the second tile on)
         for (; c + 2 <= J; c += 2) {
           next_tile_ct(c, std::integral_constant<int, 1>{}, lin_t);
           next_tile_ct(c + 1, std::integral_constant<int, 0>{}, lin_t);
         }
       } else {
-        // unmasked tiles in rounds of NS, tile c in stage c % NS (1, 2, 0 from c = 1 on)
+        // unmasked tiles in rounds of NS, tile c in stage c % NS (1, 2, 0 from the second tile on)
         static_assert(NS == 3, "the rounds below are written for a 3-stage ring");
         for (; c + NS <= J; c += NS) {
           next_tile_ct(c, std::integral_constant<int, 1>{}, lin_t);
@@ -2888,7 +2913,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
         softmax_pv(scur);
         advance();
       }
-      for (; c < ntiles; ++c) {
+      for (; c < c_hi; ++c) {
         next_tile(c, lin_t, std::true_type{});
         softmax_pv(scur);
         advance();
@@ -2915,7 +2940,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
       scur = 0;
       snext = NS - 1;
       s8 = 0;
-      for (int c = 0; c < ntiles; ++c) {
+      for (int c = c_lo; c < c_hi; ++c) {
         next_tile(c, linear, std::true_type{});
         row_top();
         if (needs_rescale()) rescale();
@@ -2926,11 +2951,26 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
     }
   }
 
+  bool piece = false;   // one of several pieces of the rows (read again: not held through the tile loops)
+  int pslot = 0;
+  if constexpr (SPLIT) {
+    int x = blockIdx.x;
+    asm volatile("" : "+s"(x));
+    piece = (a.tile_piece[x] >> 16) > 1;
+    pslot = a.tile_slot[x];
+  }
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     const float lr = group4_sum(l[rb]);
     if (!valid[rb]) continue;
-    const float inv = lr > 0.f ? 1.f / lr : 0.f;
+    float inv = lr > 0.f ? 1.f / lr : 0.f;
+    float* prow = nullptr;
+    if (SPLIT && piece) {
+      inv = 1.f;   // a piece leaves its accumulators as they are: the merge divides by the whole denominator
+      const int64_t pr = ((int64_t)pslot * gridDim.y + kvh) * PR_ROWS + (wave * RB + rb) * 16 + n;
+      if (g == 0) *reinterpret_cast<float2*>(a.part_ml + 2 * pr) = float2{m[rb], lr};
+      prow = a.part_out + pr * D + 4 * g;
+    }
     uint16_t* orow = a.out + (int64_t)(tok + t[rb]) * a.o_st + (int64_t)hq[rb] * a.o_sh + 4 * g;
 #pragma unroll
     for (int tt = 0; tt < VT; ++tt) {
@@ -2943,6 +2983,10 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
           o *= a.vs[kvh];
         }
       }
+      if (SPLIT && piece) {
+        *reinterpret_cast<f32x4*>(prow + 16 * tt) = o;
+        continue;
+      }
       u32x2 w;
       w.x = pack_bf16x2_rne(o[0], o[1]);
       w.y = pack_bf16x2_rne(o[2], o[3]);
@@ -2951,9 +2995,9 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
   }
 }
 
-template <int D>
+template <int D, bool SPLIT>
 __global__ __launch_bounds__(256, 3) void prefill_kernel(PrefillArgs a) {
-  prefill_body<D, PR_SRC_BF16>(a);
+  prefill_body<D, PR_SRC_BF16, SPLIT>(a);
 }
 
 // The same attention reading the INT8 pages themselves, in place of dequant_pages + prefill_kernel:
@@ -2961,9 +3005,57 @@ __global__ __launch_bounds__(256, 3) void prefill_kernel(PrefillArgs a) {
 // is converted in LDS. PR_SRC_I8: with dequant_pages' arithmetic, so the output is bit-identical to the
 // two-kernel path's. PR_SRC_I8_FOLD: codes converted exactly, k_scale folded into q and v_scale applied
 // to the output (one rounding of q x k_scale in place of one of code x scale per K and V element).
-template <int D, int SRC>
+template <int D, int SRC, bool SPLIT>
 __global__ __launch_bounds__(256, 3) void prefill_i8_kernel(PrefillArgs a) {
-  prefill_body<D, SRC>(a);
+  prefill_body<D, SRC, SPLIT>(a);
+}
+
+// The rows of a split work list whose keys were cut into pieces: out = sum_p 2^(m_p - M) acc_p /
+// sum_p 2^(m_p - M) l_p over the pieces p, M the largest reference maximum of a piece that saw a key of the
+// row (a piece without one has l = 0 and counts for nothing). One wavefront per row, lane p holding piece p's
+// weight (at most MAX_PREFILL_PARTS = 64 of them), lanes D / 64 channels each, four pieces' accumulators
+// requested at a time. Entry x of `merge` is (request, first row, first slot, pieces).
+constexpr int PR_MERGE_WAVES = 4;
+constexpr int MAX_PREFILL_PARTS = 64;
+template <int D>
+__global__ __launch_bounds__(WAVE * PR_MERGE_WAVES) void prefill_merge_kernel(PrefillArgs a, const int4* __restrict__ merge) {
+  constexpr int CPL = D / WAVE, UNR = 4;
+  const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int4 e = merge[blockIdx.x];
+  const int kvh = blockIdx.y, hkv = gridDim.y, lrow = blockIdx.z * PR_MERGE_WAVES + wave;
+  const int P = e.w;
+  const int64_t row0 = ((int64_t)e.z * hkv + kvh) * PR_ROWS + lrow, step = (int64_t)hkv * PR_ROWS;
+  // (rows past the request's are never read: no piece wrote them)
+  const int tok = a.cu_q[e.x], Q = a.cu_q[e.x + 1] - tok;
+  const int R = e.y + lrow, t = R / a.G;
+  if (t >= Q) return;
+  float2 ml = {-1e30f, 0.f};
+  if (lane < P) ml = *reinterpret_cast<const float2*>(a.part_ml + 2 * (row0 + lane * step));
+  const float* po = a.part_out + row0 * D + CPL * lane;
+  const bool seen = !(ml.y == 0.f);
+  const float M = wave_max(seen ? ml.x : -1e30f);
+  const float wt = seen ? __builtin_amdgcn_exp2f(ml.x - M) : 0.f;
+  const float den = wave_sum(wt * ml.y);
+  const float inv = den > 0.f ? 1.f / den : 0.f;
+  float num[CPL];
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) num[c] = 0.f;
+  for (int p0 = 0; p0 < P; p0 += UNR) {
+    float v[UNR][CPL];
+#pragma unroll
+    for (int u = 0; u < UNR; ++u)
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) v[u][c] = po[min(p0 + u, P - 1) * step * D + c];
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) {
+      const float ws = p0 + u < P ? __shfl(wt, min(p0 + u, P - 1), WAVE) : 0.f;
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) num[c] = ws != 0.f ? __builtin_fmaf(ws, v[u][c], num[c]) : num[c];
+    }
+  }
+  uint16_t* op = a.out + (int64_t)(tok + t) * a.o_st + (int64_t)(kvh * a.G + R % a.G) * a.o_sh + CPL * lane;
+  if constexpr (CPL == 2) *reinterpret_cast<uint32_t*>(op) = pack_bf16x2_rne(num[0] * inv, num[1] * inv);
+  else op[0] = (uint16_t)pack_bf16x2_rne(num[0] * inv, 0.f);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -3285,6 +3377,15 @@ namespace {
 
 // Shared by the bf16 (dequant_pages' temporary cache) and the INT8 (the pages themselves) prefill:
 // es = bytes per cache element (2 or 1); ks / vs only for the INT8 caches.
+struct PrefillSplit {   // the split work list of an _ex call; tile_piece NULL: none
+  const int32_t* tile_piece = nullptr;
+  const int32_t* tile_slot = nullptr;
+  const int32_t* merge = nullptr;
+  int64_t num_merge = 0;
+  float* part_out = nullptr;
+  float* part_ml = nullptr;
+};
+
 int prefill_launch(const char* nm, int es, const void* q, int64_t q_st, int64_t q_sh, const void* k_cache,
                    int64_t k_sb, int64_t k_sn, int64_t k_sh, const void* v_cache, int64_t v_sb, int64_t v_sn,
                    int64_t v_sh, int64_t num_blocks, int64_t block_size, int64_t num_kv_heads, int64_t head_dim,
@@ -3292,7 +3393,7 @@ int prefill_launch(const char* nm, int es, const void* q, int64_t q_st, int64_t 
                    const int32_t* block_table, int64_t bt_stride, int64_t num_q_heads, const int32_t* tile_req,
                    const int32_t* tile_row, int64_t num_tiles, int64_t rows_per_tile, double softmax_scale,
                    const float* k_scale, int64_t k_scale_cols, const float* v_scale, int64_t v_scale_cols,
-                   int64_t fold_scales, void* stream) {
+                   int64_t fold_scales, const PrefillSplit& split, void* stream) {
   if (head_dim != 64 && head_dim != 128) return fail("%s: head_dim must be 64 or 128, got %lld", nm, (long long)head_dim);
   if (block_size < 16 || !pow2(block_size)) return fail("%s: block_size must be a power of two >= 16", nm);
   if (num_kv_heads <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads || num_kv_heads > 65535)
@@ -3312,6 +3413,13 @@ int prefill_launch(const char* nm, int es, const void* q, int64_t q_st, int64_t 
   if (k_sb < 0 || v_sb < 0 || k_sn < 0 || v_sn < 0 || es * k_sb > UINT32_MAX || es * v_sb > UINT32_MAX ||
       es * block_size * k_sn > INT32_MAX || es * block_size * v_sn > INT32_MAX)
     return fail("%s: page too large for 32-bit page / slot offsets", nm);
+  if (split.tile_piece) {
+    if (!split.tile_slot || split.num_merge < 0 || split.num_merge > INT32_MAX)
+      return fail("%s: bad split work list", nm);
+    if (split.num_merge > 0 && (!split.merge || !split.part_out || !split.part_ml || !aligned16(split.merge) ||
+                                !aligned16(split.part_out) || !aligned16(split.part_ml)))
+      return fail("%s: split work list needs 16-byte aligned merge list and partial buffers", nm);
+  }
   PrefillArgs a;
   a.q = (const uint16_t*)q; a.kc = (const uint16_t*)k_cache; a.vc = (const uint16_t*)v_cache; a.out = (uint16_t*)out;
   a.cu_q = cu_seqlens_q; a.seq_lens = seq_lens; a.block_table = block_table; a.tile_req = tile_req; a.tile_row = tile_row;
@@ -3323,19 +3431,27 @@ int prefill_launch(const char* nm, int es, const void* q, int64_t q_st, int64_t 
   a.krow = (uint32_t)(es * k_sn); a.vrow = (uint32_t)(es * v_sn);
   a.contig = (k_sb == block_size * k_sn && v_sb == block_size * v_sn) ? 1 : 0;
   a.ks = k_scale; a.vs = v_scale; a.ks_pc = k_scale_cols > 1; a.vs_pc = v_scale_cols > 1;
+  a.tile_piece = split.tile_piece; a.tile_slot = split.tile_slot; a.part_out = split.part_out; a.part_ml = split.part_ml;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)num_tiles, (unsigned)num_kv_heads);
-  if (es == 1 && fold_scales) {
-    if (head_dim == 128) hipLaunchKernelGGL((prefill_i8_kernel<128, PR_SRC_I8_FOLD>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((prefill_i8_kernel<64, PR_SRC_I8_FOLD>), grid, dim3(256), 0, st, a);
-  } else if (es == 1) {
-    if (head_dim == 128) hipLaunchKernelGGL((prefill_i8_kernel<128, PR_SRC_I8>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((prefill_i8_kernel<64, PR_SRC_I8>), grid, dim3(256), 0, st, a);
-  } else {
-    if (head_dim == 128) hipLaunchKernelGGL(prefill_kernel<128>, grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(prefill_kernel<64>, grid, dim3(256), 0, st, a);
-  }
-  return launched(nm);
+  auto go = [&](auto d_t, auto split_t) {
+    constexpr int D = decltype(d_t)::value;
+    constexpr bool SPLIT = decltype(split_t)::value;
+    if (es == 2) hipLaunchKernelGGL((prefill_kernel<D, SPLIT>), grid, dim3(256), 0, st, a);
+    else if (fold_scales) hipLaunchKernelGGL((prefill_i8_kernel<D, PR_SRC_I8_FOLD, SPLIT>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((prefill_i8_kernel<D, PR_SRC_I8, SPLIT>), grid, dim3(256), 0, st, a);
+  };
+  const std::integral_constant<int, 128> d128;
+  const std::integral_constant<int, 64> d64;
+  if (split.tile_piece) head_dim == 128 ? go(d128, std::true_type{}) : go(d64, std::true_type{});
+  else head_dim == 128 ? go(d128, std::false_type{}) : go(d64, std::false_type{});
+  const int rc = launched(nm);
+  if (rc != KVQ_OK || !split.tile_piece || split.num_merge == 0) return rc;
+  const dim3 mgrid((unsigned)split.num_merge, (unsigned)num_kv_heads, PR_ROWS / PR_MERGE_WAVES);
+  const int4* ml = reinterpret_cast<const int4*>(split.merge);
+  if (head_dim == 128) hipLaunchKernelGGL(prefill_merge_kernel<128>, mgrid, dim3(WAVE * PR_MERGE_WAVES), 0, st, a, ml);
+  else hipLaunchKernelGGL(prefill_merge_kernel<64>, mgrid, dim3(WAVE * PR_MERGE_WAVES), 0, st, a, ml);
+  return launched("prefill_merge");
 }
 
 }  // namespace
@@ -3353,7 +3469,23 @@ int kvq_paged_prefill_attention(const void* q, int64_t q_st, int64_t q_sh, const
   return prefill_launch("paged_prefill_attention", 2, q, q_st, q_sh, k_cache, k_sb, k_sn, k_sh, v_cache, v_sb, v_sn,
                         v_sh, num_blocks, block_size, num_kv_heads, head_dim, out, o_st, o_sh, cu_seqlens_q,
                         seq_lens, block_table, bt_stride, num_q_heads, tile_req, tile_row, num_tiles, rows_per_tile,
-                        softmax_scale, nullptr, 1, nullptr, 1, 0, stream);
+                        softmax_scale, nullptr, 1, nullptr, 1, 0, PrefillSplit{}, stream);
+}
+
+int kvq_paged_prefill_attention_ex(const void* q, int64_t q_st, int64_t q_sh, const void* k_cache, int64_t k_sb,
+                                   int64_t k_sn, int64_t k_sh, const void* v_cache, int64_t v_sb, int64_t v_sn,
+                                   int64_t v_sh, int64_t num_blocks, int64_t block_size, int64_t num_kv_heads,
+                                   int64_t head_dim, void* out, int64_t o_st, int64_t o_sh,
+                                   const int32_t* cu_seqlens_q, const int32_t* seq_lens, const int32_t* block_table,
+                                   int64_t bt_stride, int64_t num_q_heads, const int32_t* tile_req,
+                                   const int32_t* tile_row, int64_t num_tiles, int64_t rows_per_tile,
+                                   double softmax_scale, const int32_t* tile_piece, const int32_t* tile_slot,
+                                   const int32_t* merge, int64_t num_merge, float* part_out, float* part_ml, void* stream) {
+  return prefill_launch("paged_prefill_attention_ex", 2, q, q_st, q_sh, k_cache, k_sb, k_sn, k_sh, v_cache, v_sb, v_sn,
+                        v_sh, num_blocks, block_size, num_kv_heads, head_dim, out, o_st, o_sh, cu_seqlens_q,
+                        seq_lens, block_table, bt_stride, num_q_heads, tile_req, tile_row, num_tiles, rows_per_tile,
+                        softmax_scale, nullptr, 1, nullptr, 1, 0,
+                        PrefillSplit{tile_piece, tile_slot, merge, num_merge, part_out, part_ml}, stream);
 }
 
 int kvq_int8_prefill_attention(const void* q, int64_t q_st, int64_t q_sh, const int8_t* k_cache, int64_t k_sb,
@@ -3369,7 +3501,26 @@ int kvq_int8_prefill_attention(const void* q, int64_t q_st, int64_t q_sh, const 
   return prefill_launch("int8_prefill_attention", 1, q, q_st, q_sh, k_cache, k_sb, k_sn, k_sh, v_cache, v_sb, v_sn,
                         v_sh, num_blocks, block_size, num_kv_heads, head_dim, out, o_st, o_sh, cu_seqlens_q,
                         seq_lens, block_table, bt_stride, num_q_heads, tile_req, tile_row, num_tiles, rows_per_tile,
-                        softmax_scale, k_scale, k_scale_cols, v_scale, v_scale_cols, fold_scales, stream);
+                        softmax_scale, k_scale, k_scale_cols, v_scale, v_scale_cols, fold_scales, PrefillSplit{}, stream);
+}
+
+int kvq_int8_prefill_attention_ex(const void* q, int64_t q_st, int64_t q_sh, const int8_t* k_cache, int64_t k_sb,
+                                  int64_t k_sn, int64_t k_sh, const int8_t* v_cache, int64_t v_sb, int64_t v_sn,
+                                  int64_t v_sh, int64_t num_blocks, int64_t block_size, int64_t num_kv_heads,
+                                  int64_t head_dim, void* out, int64_t o_st, int64_t o_sh,
+                                  const int32_t* cu_seqlens_q, const int32_t* seq_lens, const int32_t* block_table,
+                                  int64_t bt_stride, int64_t num_q_heads, const int32_t* tile_req,
+                                  const int32_t* tile_row, int64_t num_tiles, int64_t rows_per_tile,
+                                  double softmax_scale, const float* k_scale, int64_t k_scale_cols,
+                                  const float* v_scale, int64_t v_scale_cols, int64_t fold_scales,
+                                  const int32_t* tile_piece, const int32_t* tile_slot, const int32_t* merge,
+                                  int64_t num_merge, float* part_out, float* part_ml, void* stream) {
+  if (fold_scales != 0 && fold_scales != 1) return fail("int8_prefill_attention_ex: fold_scales must be 0 or 1");
+  return prefill_launch("int8_prefill_attention_ex", 1, q, q_st, q_sh, k_cache, k_sb, k_sn, k_sh, v_cache, v_sb, v_sn,
+                        v_sh, num_blocks, block_size, num_kv_heads, head_dim, out, o_st, o_sh, cu_seqlens_q,
+                        seq_lens, block_table, bt_stride, num_q_heads, tile_req, tile_row, num_tiles, rows_per_tile,
+                        softmax_scale, k_scale, k_scale_cols, v_scale, v_scale_cols, fold_scales,
+                        PrefillSplit{tile_piece, tile_slot, merge, num_merge, part_out, part_ml}, stream);
 }
 
 int kvq_set_attention_events(void* start, void* stop) {
@@ -3434,9 +3585,11 @@ int kvq_stream_scatter(const void* key, int64_t key_st, int64_t key_sh, const vo
   return launched("stream_scatter");
 }
 
-int kvq_abi_version(void) { return 11; }
+int kvq_abi_version(void) { return 12; }
 
 int kvq_prefill_rows_per_tile(void) { return PR_ROWS; }
+
+int kvq_prefill_max_parts(void) { return MAX_PREFILL_PARTS; }
 
 int kvq_quant_cache(const void* key, int64_t key_st, int64_t key_sh, const void* value, int64_t val_st,
                     int64_t val_sh, int8_t* k_cache, int64_t kc_sb, int64_t kc_sn, int64_t kc_sh, int8_t* v_cache,

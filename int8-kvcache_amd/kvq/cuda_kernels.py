@@ -191,7 +191,9 @@ class _Ext:
                      ks.data_ptr(), kcols, vs.data_ptr(), vcols, _stream(kc))
 
     # consumer of the temporary cache: in place of flash_attn_varlen_func (kvq/cuda_kernels.py:128-130)
-    def paged_prefill_attention(self, q, kt, vt, out, cu_q, seq_lens, block_table, tile_req, tile_row, softmax_scale):
+    # (split = LongPlan.pieces' list in place of the whole rows' tile_req / tile_row, with its buffers)
+    def paged_prefill_attention(self, q, kt, vt, out, cu_q, seq_lens, block_table, tile_req, tile_row, softmax_scale,
+                                split=None):
         n = tile_req.shape[0]
         if n == 0:
             return
@@ -206,17 +208,36 @@ class _Ext:
             _check(t.dtype == torch.int32, f"paged_prefill_attention: {nm} must be int32")
         _check(block_table.stride(-1) == 1 and tile_row.shape[0] == n, "paged_prefill_attention: index layout")
         P, bs, Hkv, d = kt.shape
-        _native.call("kvq_paged_prefill_attention", q.data_ptr(), q.stride(0), q.stride(1), kt.data_ptr(), kt.stride(0),
-                     kt.stride(1), kt.stride(2), vt.data_ptr(), vt.stride(0), vt.stride(1), vt.stride(2), P, bs, Hkv, d,
-                     out.data_ptr(), out.stride(0), out.stride(1), cu_q.data_ptr(), seq_lens.data_ptr(),
-                     block_table.data_ptr(), block_table.stride(0), q.shape[1], tile_req.data_ptr(),
-                     tile_row.data_ptr(), n, self.prefill_rows, float(softmax_scale), _stream(q))
+        args = [q.data_ptr(), q.stride(0), q.stride(1), kt.data_ptr(), kt.stride(0),
+                kt.stride(1), kt.stride(2), vt.data_ptr(), vt.stride(0), vt.stride(1), vt.stride(2), P, bs, Hkv, d,
+                out.data_ptr(), out.stride(0), out.stride(1), cu_q.data_ptr(), seq_lens.data_ptr(),
+                block_table.data_ptr(), block_table.stride(0), q.shape[1], tile_req.data_ptr(),
+                tile_row.data_ptr(), n, self.prefill_rows, float(softmax_scale)]
+        if split is None:
+            _native.call("kvq_paged_prefill_attention", *args, _stream(q))
+        else:
+            _native.call("kvq_paged_prefill_attention_ex", *args, *self._split_args(split, n, Hkv, d), _stream(q))
+
+    def _split_args(self, split, n, hkv, d):
+        """The C arguments of a split work list: tile_piece, tile_slot, merge, num_merge, part_out, part_ml."""
+        tile_piece, tile_slot, merge, part_out, part_ml = split
+        rows = self.prefill_rows
+        for t in (tile_piece, tile_slot, merge):
+            _check(t.dtype == torch.int32 and t.is_contiguous(), "prefill split: lists must be contiguous int32")
+        for t in (part_out, part_ml):
+            _check(t.dtype == torch.float32 and t.is_contiguous(), "prefill split: partials must be contiguous float32")
+        _check_cuda("prefill split", tile_piece, tile_slot, merge, part_out, part_ml)
+        _check(tile_piece.shape == (n,) and tile_slot.shape == (n,) and merge.dim() == 2 and merge.shape[1] == 4 and
+               tuple(part_out.shape[1:]) == (hkv, rows, d) and tuple(part_ml.shape) == (part_out.shape[0], hkv, rows, 2),
+               "prefill split: list and buffer shapes")
+        return (tile_piece.data_ptr(), tile_slot.data_ptr(), merge.data_ptr(), merge.shape[0], part_out.data_ptr(),
+                part_ml.data_ptr())
 
     # the same attention read straight from the INT8 pages, in place of dequant_pages + the call above
     # (no counterpart in the reference, which always dequantizes first: kvq/cuda_kernels.py:106-131).
     # fold=False: bit-identical to that pair; True: scales folded into q and the output (faster)
     def int8_prefill_attention(self, q, kc, vc, out, cu_q, seq_lens, block_table, tile_req, tile_row, softmax_scale,
-                               ks, vs, fold=False):
+                               ks, vs, fold=False, split=None):
         n = tile_req.shape[0]
         if n == 0:
             return
@@ -233,17 +254,26 @@ class _Ext:
         nb, bs, Hkv, d = kc.shape
         kcols = _scale_cols(ks, "int8_prefill_attention k_scale", Hkv, d)
         vcols = _scale_cols(vs, "int8_prefill_attention v_scale", Hkv, d)
-        _native.call("kvq_int8_prefill_attention", q.data_ptr(), q.stride(0), q.stride(1), kc.data_ptr(), kc.stride(0),
-                     kc.stride(1), kc.stride(2), vc.data_ptr(), vc.stride(0), vc.stride(1), vc.stride(2), nb, bs, Hkv,
-                     d, out.data_ptr(), out.stride(0), out.stride(1), cu_q.data_ptr(), seq_lens.data_ptr(),
-                     block_table.data_ptr(), block_table.stride(0), q.shape[1], tile_req.data_ptr(),
-                     tile_row.data_ptr(), n, self.prefill_rows, float(softmax_scale), ks.data_ptr(), kcols,
-                     vs.data_ptr(), vcols, int(bool(fold)), _stream(q))
+        args = [q.data_ptr(), q.stride(0), q.stride(1), kc.data_ptr(), kc.stride(0),
+                kc.stride(1), kc.stride(2), vc.data_ptr(), vc.stride(0), vc.stride(1), vc.stride(2), nb, bs, Hkv,
+                d, out.data_ptr(), out.stride(0), out.stride(1), cu_q.data_ptr(), seq_lens.data_ptr(),
+                block_table.data_ptr(), block_table.stride(0), q.shape[1], tile_req.data_ptr(),
+                tile_row.data_ptr(), n, self.prefill_rows, float(softmax_scale), ks.data_ptr(), kcols,
+                vs.data_ptr(), vcols, int(bool(fold))]
+        if split is None:
+            _native.call("kvq_int8_prefill_attention", *args, _stream(q))
+        else:
+            _native.call("kvq_int8_prefill_attention_ex", *args, *self._split_args(split, n, Hkv, d), _stream(q))
 
     @property
     def prefill_rows(self):
         """(token, q head) rows per work-list entry of the prefill kernel."""
         return int(_native.load().kvq_prefill_rows_per_tile())
+
+    @property
+    def prefill_max_parts(self):
+        """Most pieces an entry's keys may be cut into."""
+        return int(_native.load().kvq_prefill_max_parts())
 
 
 def ext():
@@ -366,6 +396,7 @@ class LongPlan:
     long_seq: np.ndarray = None
     _gpu: tuple = None
     _tiles: dict = None
+    _work: dict = None
 
     def gpu(self, device):
         if self._gpu is None:
@@ -381,17 +412,134 @@ class LongPlan:
         if self._tiles is None:
             self._tiles = {}
         if (group, rows) not in self._tiles:
-            req, row, cost = [], [], []
-            for r, qn, sl in zip(self.long_req.tolist(), self.long_qlen.tolist(), self.long_seq.tolist()):
-                for r0 in range(0, qn * group, rows):
-                    t_last = min(qn - 1, (r0 + rows - 1) // group)
-                    req.append(r)
-                    row.append(r0)
-                    cost.append(sl - qn + 1 + t_last)
-            order = np.argsort(-np.asarray(cost, dtype=np.int64), kind="stable")
-            self._tiles[(group, rows)] = tuple(torch.from_numpy(np.asarray(x, dtype=np.int32)[order]).to(device)
+            req, row, cost = self._row_tiles(group, rows)
+            order = np.argsort(-cost, kind="stable")
+            self._tiles[(group, rows)] = tuple(torch.from_numpy(x.astype(np.int32)[order]).to(device)
                                                for x in (req, row))
         return self._tiles[(group, rows)]
+
+    def _row_tiles(self, group, rows):
+        """(request, first row, keys its last row reads) of every `rows` (token, q head) rows, int64."""
+        n = (self.long_qlen * group + rows - 1) // rows
+        at = np.repeat(np.arange(n.shape[0]), n)
+        row = (np.arange(at.shape[0]) - np.repeat(np.cumsum(n) - n, n)) * rows
+        last = np.minimum(self.long_qlen[at] - 1, (row + rows - 1) // group)
+        return self.long_req[at].astype(np.int64), row, self.long_seq[at] - self.long_qlen[at] + 1 + last
+
+    def work(self, group, hkv, d, device):
+        """The prefill call's work list on the device (PrefillWork): `tiles`, the longest rows' keys cut into
+        pieces where that pays (split_rows), and whether the call reads the INT8 pages itself. Built on the
+        host, copied once per plan and shape."""
+        if self._work is None:
+            self._work = {}
+        if (group, hkv, d) not in self._work:
+            rows = ext().prefill_rows
+            req, row, keys = self._row_tiles(group, rows)
+            tiles = np.maximum((keys + PREFILL_TILE - 1) // PREFILL_TILE, 1)
+            lists = split_rows(req, row, tiles, hkv, d, one_pass_fill(device), ext().prefill_max_parts)
+            if lists is None:
+                order = np.argsort(-keys, kind="stable")
+                lists, longest, slots = (req[order], row[order]), int(tiles.max(initial=0)), 0
+            else:
+                longest, slots = lists[5:]
+                lists = (lists[4], *lists[:4])   # the 16-byte merge entries first
+            flat = torch.from_numpy(np.concatenate([x.astype(np.int32).reshape(-1) for x in lists])).to(device)
+            at, views = 0, []
+            for x in lists:
+                views.append(flat[at:at + x.size].view(x.shape))
+                at += x.size
+            pages = self.src_req.shape[0] * self.block_size * hkv * d
+            direct = direct_pays(longest, d, pages)
+            self._work[(group, hkv, d)] = (PrefillWork(*views, None, None, None, 0, direct) if len(views) == 2 else
+                                           PrefillWork(views[1], views[2], views[3], views[4], views[0], slots, direct))
+        return self._work[(group, hkv, d)]
+
+
+@dataclass
+class PrefillWork:
+    """One prefill call's work list: (request, first row) of each entry and, where rows were cut into pieces,
+    each entry's piece and slot and the list of cut rows to merge (kvq_paged_prefill_attention_ex)."""
+    tile_req: torch.Tensor
+    tile_row: torch.Tensor
+    tile_piece: torch.Tensor
+    tile_slot: torch.Tensor
+    merge: torch.Tensor
+    slots: int
+    direct: bool                # read the INT8 pages (same output bits) instead of dequantizing them first
+
+    def split(self, hkv, rows, d):
+        """The split arguments of the prefill calls with fresh partial buffers, or None."""
+        if self.tile_piece is None:
+            return None
+        device = self.tile_req.device
+        return (self.tile_piece, self.tile_slot, self.merge,
+                torch.empty(self.slots, hkv, rows, d, dtype=torch.float32, device=device),
+                torch.empty(self.slots, hkv, rows, 2, dtype=torch.float32, device=device))
+
+
+PREFILL_TILE = 32          # keys per tile of the prefill kernel
+PREFILL_MIN_PIECE = 4      # shortest piece, in tiles: a shorter one costs its start and merge more than it saves
+PREFILL_PER_CU = 2         # pieces per CU a split work list may hold
+PREFILL_WHOLE = 1.5        # workgroups of whole rows per CU from which nothing is cut
+# us, measured at head_dim 128 (a tile costs 0.7 of it at 64, a piece half): a tile of a workgroup alone on its CU, the same with two
+# workgroups per CU, the same when the INT8 pages are converted in the kernel (beyond the first), the merge
+# launch, and a piece's partials (66 KB per kv head, written and read)
+TILE_US, TILE2_US, TILE_DIRECT_US, MERGE_US, PIECE_US = 0.6, 0.85, 0.38, 4.0, 0.02
+DEQUANT_US, DEQUANT_ELEMS_PER_US = 4.0, 0.85e6   # dequant_pages: its launch, K + V elements (6 bytes) per us
+
+
+def _tile_unit(d):
+    return 1.0 if d == 128 else 0.7
+
+
+def split_rows(req, row, tiles, hkv, d, fill, max_parts):
+    """Cut the long rows of a prefill work list (request, first row, key tiles; one workgroup per entry and kv
+    head) into pieces of key tiles: (req, row, piece | pieces << 16, slot, merge [cut rows, 4], longest piece,
+    slots), heaviest pieces first, or None where nothing is cut.
+
+    A workgroup walks its tiles one after another, so few rows over many keys leave most CUs idle. The pieces
+    are the shortest that keep the list within PREFILL_PER_CU workgroups per CU (all resident, the CUs evenly
+    loaded); a third per CU adds partials and merging without time (graph, 28 / 4 heads, 512 tokens of 8,192
+    keys: whole 169 us, 1 / 2 / 3 pieces per CU 106 / 90 / 103 us; 16 tokens of 16,384: 322 -> 39 us). Cut only
+    where the tiles saved are worth the partials and the merge: 1,024 tokens of 1,024 whole 34 us, cut 38; 256 of
+    256 16 and 19; 700 of 3,000 71 and 56; 128 of 1,000 31 and 28. From PREFILL_WHOLE workgroups per CU on the
+    rows balance among themselves: 448 workgroups (2,048 tokens from the start) 62 us whole, 64 cut."""
+    if req.shape[0] * hkv >= PREFILL_WHOLE * fill or req.shape[0] == 0:
+        return None
+    lo, hi = PREFILL_MIN_PIECE, max(PREFILL_MIN_PIECE, int(tiles.max()))
+    while lo < hi:             # the shortest piece length that fits
+        mid = (lo + hi) // 2
+        if int(((tiles + mid - 1) // mid).sum()) * hkv <= PREFILL_PER_CU * fill:
+            hi = mid
+        else:
+            lo = mid + 1
+    parts = np.minimum((tiles + lo - 1) // lo, max_parts)
+    cut = parts > 1
+    pieces = int(parts.sum()) * hkv
+    longest = int(((tiles + parts - 1) // parts).max())
+    whole_us = TILE_US * _tile_unit(d) * int(tiles.max())
+    cut_us = (TILE2_US if pieces > fill else TILE_US) * _tile_unit(d) * longest + MERGE_US + PIECE_US * d / 128 * pieces
+    if not cut.any() or cut_us >= whole_us:
+        return None
+    at = np.repeat(np.arange(parts.shape[0]), parts)
+    part = np.arange(at.shape[0]) - np.repeat(np.cumsum(parts) - parts, parts)
+    held = np.where(cut, parts, 0)
+    first = np.cumsum(held) - held                       # slot of a cut entry's piece 0
+    order = np.argsort(-(tiles[at] // parts[at]), kind="stable")
+    merge = np.stack([req[cut], row[cut], first[cut], parts[cut]], 1)
+    slot = np.where(cut[at], first[at] + part, 0)
+    return (req[at][order], row[at][order], (part | parts[at] << 16)[order], slot[order], merge, longest,
+            int(held.sum()))
+
+
+def direct_pays(longest, d, elems):
+    """Whether the prefill reads the INT8 pages itself (int8_prefill_attention, the same output bits) instead of
+    dequantizing `elems` K (and as many V) elements first: converting a tile in the kernel costs each workgroup,
+    whose longest has `longest` tiles, more than reading it as bf16, and saves the dequantization's launch, pass
+    over the pages and temporary cache. Graph, 28 / 4 heads, two kernels and direct: 64 tokens of 8,192 keys 37.4
+    and 36.0 us, 16 of 16,384 39.2 and 30.8, 256 of 256 16.2 and 15.4; 512 of 8,192 90 and 108, 1,024 of 1,024
+    34 and 40; 300 of 12,000 (16 / 16 heads, d64) 57 and 51."""
+    return TILE_DIRECT_US * _tile_unit(d) * longest < DEQUANT_US + elems / DEQUANT_ELEMS_PER_US
 
 
 def plan_long(query_start_loc_cpu, seq_lens_cpu, block_size):
@@ -429,29 +577,34 @@ def long_attention(q, k_cache, v_cache, out, cu_seqlens_q, seq_lens, block_table
     short requests are left to decode_attention. The key counts are read on the device (seq_lens), the
     plan's host lengths only size the temporary cache and order the work. KVQ_DEBUG_DUMP=path saves the
     prefill call's metadata there first (kvq.debug_dump; the reference's dump, kvq/cuda_kernels.py:123-127).
-    KVQ_PREFILL_DIRECT (read at every call): 1 = one kernel reads the INT8 pages itself instead
-    (int8_prefill_attention) -- no temporary cache, bit-identical output; fold = the same with the scales
-    folded into q and the output (faster, not bit-identical); 0 (default) = the two kernels."""
+    Rows of many keys may be cut into pieces and merged (LongPlan.work). KVQ_PREFILL_DIRECT (read at every
+    call): 1 = one kernel reads the INT8 pages itself instead (int8_prefill_attention) -- no temporary cache,
+    bit-identical output; fold = the same with the scales folded into q and the output (faster, not
+    bit-identical); 0 = the two kernels; unset = 1 or 0, whichever is faster (direct_pays)."""
     bs, h, d = k_cache.shape[1:]
     _check(bs == plan.block_size, f"block size {bs} != plan block size {plan.block_size}")
-    tile_req, tile_row = plan.tiles(q.shape[1] // h, q.device)
+    work = plan.work(q.shape[1] // h, h, d, q.device)
+    tile_req, tile_row = work.tile_req, work.tile_row
     kt_shape = (plan.src_req.shape[0], bs, h, d)
     if os.environ.get("KVQ_DEBUG_DUMP"):  # the prefill call's metadata, for an offline replay (kvq.debug_dump)
         from . import debug_dump
         debug_dump.dump_long_call(os.environ["KVQ_DEBUG_DUMP"], q, out, cu_seqlens_q, seq_lens, plan, kt_shape,
-                                  tile_req, tile_row, max_query_len, ext().prefill_rows, softmax_scale)
-    direct = os.environ.get("KVQ_PREFILL_DIRECT", "0")
+                                  *plan.tiles(q.shape[1] // h, q.device), max_query_len, ext().prefill_rows,
+                                  softmax_scale)
+    direct = os.environ.get("KVQ_PREFILL_DIRECT") or ("1" if work.direct else "0")
+    split = work.split(h, ext().prefill_rows, d) if direct in ("0", "1", "fold") else None
     if direct in ("1", "fold"):
         # the INT8 pages read directly: no temporary cache ("1": same output bits; "fold": scales folded)
         ext().int8_prefill_attention(q, k_cache, v_cache, out, cu_seqlens_q, seq_lens, block_table, tile_req,
-                                     tile_row, softmax_scale, static["k_scale"], static["v_scale"], direct == "fold")
+                                     tile_row, softmax_scale, static["k_scale"], static["v_scale"], direct == "fold", split)
         return out
     _check(direct == "0", f"KVQ_PREFILL_DIRECT must be 0, 1 or fold, got {direct!r}")
     src_req, src_j, bt_tmp = plan.gpu(q.device)
     kt = torch.empty(kt_shape, dtype=q.dtype, device=q.device)
     vt = torch.empty_like(kt)
     ext().dequant_pages(k_cache, v_cache, kt, vt, block_table, src_req, src_j, static["k_scale"], static["v_scale"])
-    ext().paged_prefill_attention(q, kt, vt, out, cu_seqlens_q, seq_lens, bt_tmp, tile_req, tile_row, softmax_scale)
+    ext().paged_prefill_attention(q, kt, vt, out, cu_seqlens_q, seq_lens, bt_tmp, tile_req, tile_row, softmax_scale,
+                                  split)
     return out
 
 

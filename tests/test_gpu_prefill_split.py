@@ -1,0 +1,98 @@
+"""The prefill kernels with a split work list (kvq_paged_prefill_attention_ex, kvq_int8_prefill_attention_ex):
+rows' keys cut into pieces and merged. Checked against fp32 attention over the same pages at the bar of
+test_gpu_prefill.py; the bf16 and INT8 sources cut alike must agree bit for bit."""
+import numpy as np
+import pytest
+import torch
+from conftest import nan_like, record
+
+from oracle import kvq_oracle as O
+from kvq import cuda_kernels as ck
+from test_gpu_kernels import dev
+from test_gpu_prefill import _reference, _temp_cache
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _split(plan, group, hkv, d, parts):
+    """A work list that cuts every row tile into exactly `parts` pieces (also more than it has tiles)."""
+    rows = ck.ext().prefill_rows
+    req, row, _ = plan._row_tiles(group, rows)
+    n = req.shape[0]
+    at = np.repeat(np.arange(n), parts)
+    part = np.arange(n * parts) % parts
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x, dtype=np.int32)).to(DEV)  # noqa: E731
+    merge = np.stack([req, row, np.arange(n) * parts, np.full(n, parts)], 1) if parts > 1 else np.zeros((0, 4))
+    nan = float("nan")
+    return t(req[at]), t(row[at]), (t(part | parts << 16), t(np.arange(n * parts)), t(merge),
+                                    torch.full((n * parts, hkv, rows, d), nan, device=DEV),
+                                    torch.full((n * parts, hkv, rows, 2), nan, device=DEV))
+
+
+@pytest.mark.parametrize("shape", [(28, 4, 128), (14, 2, 64)])
+@pytest.mark.parametrize("parts", [1, 2, 3, 7, 64])
+@pytest.mark.parametrize("jump", [False, True])
+def test_split_prefill_matches_fp32_reference(shape, parts, jump):
+    """Pieces of one tile, of none (64 pieces of rows with 4 tiles) and of several; with `jump`, keys far past
+    their piece's first tile whose scores send that piece alone to the rescaling pass."""
+    hq, hkv, d = shape
+    q_lens, seq_lens = [100, 3, 37, 9, 200], [100, 50, 517, 2000, 1000]
+    cu, plan, kt, vt = _temp_cache(q_lens, seq_lens, hkv, d, 16, seed=hq + parts)
+    T = int(cu[-1])
+    q = (torch.randn(T, hq, d, generator=torch.Generator().manual_seed(1)) * 2).to(torch.bfloat16)
+    if jump:
+        q = (q.float() * 0.5 + 0.5).to(torch.bfloat16)
+        first = {r: p for p, r in reversed(list(enumerate(plan.src_req.tolist())))}
+        for r, key in ((2, 250), (3, 1990), (4, 850)):
+            kt[first[r] + key // 16, key % 16] = 60.0
+    scale = d ** -0.5
+    out = nan_like(q.to(DEV))
+    _, _, bt = plan.gpu(DEV)
+    tile_req, tile_row, split = _split(plan, hq // hkv, hkv, d, parts)
+    ck.ext().paged_prefill_attention(q.to(DEV), kt.to(DEV), vt.to(DEV), out, cu.to(DEV),
+                                     torch.tensor(seq_lens, dtype=torch.int32, device=DEV), bt, tile_req, tile_row, scale,
+                                     split)
+    out = out.cpu()
+    ref = _reference(q, kt, vt, cu, seq_lens, plan, scale)
+    got = torch.stack([out[int(cu[r]) + t] for (r, t) in ref]).float()
+    err = O.compare(torch.stack(list(ref.values())), got)
+    record("prefill_split", shape=list(shape), parts=parts, jump=jump, **err)
+    assert torch.isfinite(got).all() and err["max_abs"] <= 2e-2 and err["mean_abs"] <= 2e-3 and err["rel_l2"] < 1e-2, err
+    assert torch.isnan(out[int(cu[1]):int(cu[2])].float()).all()          # the short request's rows
+
+
+@pytest.mark.parametrize("d,layout", [(128, "pages"), (128, "consecutive"), (64, "pages")])
+@pytest.mark.parametrize("upper", [0, 300])
+def test_split_direct_prefill_bit_identical(d, layout, upper, monkeypatch):
+    """long_attention with its own split: few rows over many keys, pages in random order or consecutive (read
+    without the block table, from a piece's first page on), host lengths that overstate the keys (trailing
+    pieces find fewer or no tiles); both sources bit for bit, and the split against the whole rows."""
+    hq, hkv, bs = (28, 4, 16) if d == 128 else (14, 2, 32)
+    q_lens, seq_lens = [20, 1, 64], [3001, 40, 2100]
+    g = torch.Generator().manual_seed(5)
+    width = [-(-(n + upper) // bs) for n in seq_lens]
+    nb = sum(width) + 4
+    kq = torch.randint(-127, 128, (nb, bs, hkv, d), generator=g, dtype=torch.int8)
+    vq = torch.randint(-127, 128, (nb, bs, hkv, d), generator=g, dtype=torch.int8)
+    ids = torch.arange(nb) if layout == "consecutive" else torch.randperm(nb, generator=g)
+    bt = torch.zeros(3, max(width), dtype=torch.int32)
+    for r, n in enumerate(width):
+        bt[r, :n] = ids[sum(width[:r]):sum(width[:r]) + n]
+    st = {"k_scale": torch.rand(hkv, d, generator=g) * 0.02 + 1e-3, "v_scale": torch.rand(hkv, d, generator=g) * 0.02}
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(q_lens)]), dtype=torch.int32)
+    sl = torch.tensor(seq_lens, dtype=torch.int32)
+    q = torch.randn(int(cu[-1]), hq, d, generator=g).to(torch.bfloat16)
+    outs = {}
+    for mode, whole in (("0", 1.5), ("1", 1.5), ("0", 0)):
+        monkeypatch.setenv("KVQ_PREFILL_DIRECT", mode)
+        monkeypatch.setattr(ck, "PREFILL_WHOLE", whole)
+        plan = ck.plan_long(cu, sl + upper, bs)
+        assert (plan.work(hq // hkv, hkv, d, torch.device(DEV)).tile_piece is not None) == (whole > 0)
+        out = nan_like(dev(q))
+        ck.long_attention(dev(q), dev(kq), dev(vq), out, dev(cu), dev(sl), dev(bt), 64, plan, d ** -0.5, dev(st))
+        outs[mode, whole] = out.cpu()
+    long_rows = torch.repeat_interleave(torch.tensor(q_lens) > ck.SHORT_Q, torch.tensor(q_lens))
+    assert torch.equal(outs["0", 1.5].view(torch.int16), outs["1", 1.5].view(torch.int16))
+    err = O.compare(outs["0", 0][long_rows], outs["0", 1.5][long_rows])
+    assert err["max_abs"] <= 2e-2 and err["rel_l2"] < 5e-3, err            # bf16 P and output, sums in another order

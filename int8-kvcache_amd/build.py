@@ -1,11 +1,14 @@
-"""Build the in-tree HIP library libkvq_int8.so for gfx950 (hipcc, no JIT cache).
+"""Build the in-tree HIP library libkvq_int8.so for gfx950 (hipcc, no JIT cache) and the CPython module
+_torch_calls.so that calls it with torch tensors (host code).
 
-Run as a script (python int8-kvcache_amd/build.py) or through __graft_entry__.build(). The library
-lands next to this file's kvq/ package so that it travels with the source tree.
+Run as a script (python int8-kvcache_amd/build.py) or through __graft_entry__.build(). Both land next to
+this file's kvq/ package so that they travel with the source tree.
 """
+import importlib.util
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 SRC = os.path.join(HERE, "csrc", "kvq_int8.hip")
@@ -21,15 +24,34 @@ FLAGS = [
 ]
 
 
+CALLS_SRC = os.path.join(HERE, "csrc", "torch_calls.cpp")
+CALLS_OUT = os.path.join(HERE, "kvq", "_torch_calls.so")
+CXX = os.environ.get("KVQ_CXX", "/opt/rocm/bin/amdclang++")
+
+
+def _calls_flags():
+    torch_dir = os.path.dirname(importlib.util.find_spec("torch").origin)
+    return ["-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-I{torch_dir}/include", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}",
+            f"-L{torch_dir}/lib", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+
+
 def build(verbose=False):
-    tmp = OUT + ".tmp"
-    cmd = [HIPCC, *FLAGS, SRC, "-o", tmp]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({res.returncode}):\n{res.stderr[-4000:]}")
-    os.replace(tmp, OUT)
+    jobs = []
+    for cmd, out in (([HIPCC, *FLAGS, SRC], OUT), ([CXX, CALLS_SRC, *_calls_flags()], CALLS_OUT)):
+        cmd = [*cmd, "-o", out + ".tmp"]
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        jobs.append((subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True), out))
+    failed = []
+    for job, out in jobs:
+        text = job.communicate()[0]
+        if job.returncode != 0:
+            failed.append(f"building {os.path.basename(out)} failed ({job.returncode}):\n{text[-4000:]}")
+        else:
+            os.replace(out + ".tmp", out)
+    if failed:
+        raise RuntimeError("\n".join(failed))
     return OUT
 
 

@@ -24,6 +24,7 @@
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
+#include <unistd.h>
 
 #include <algorithm>
 #include <cstdarg>
@@ -3224,16 +3225,36 @@ int log2i(int64_t x) {
   while ((int64_t(1) << r) < x) ++r;
   return r;
 }
+// The attention's tuning variables, read at every call in one pass over the environment (a getenv each is a pass
+// each: about 2 us of a call's host time together).
+struct Tuning {
+  const char *prefetch = nullptr, *lds_prefetch = nullptr, *v32_ring = nullptr, *v32_ksplit = nullptr, *ksplit = nullptr,
+             *rows32 = nullptr, *xcd_order = nullptr, *plan_fast_max = nullptr, *lds_ring = nullptr, *seg_cost = nullptr;
+};
+Tuning read_tuning() {
+  Tuning t;
+  const struct {
+    const char* name;
+    const char** to;
+  } known[] = {{"PREFETCH=", &t.prefetch}, {"LDS_PREFETCH=", &t.lds_prefetch}, {"V32_RING=", &t.v32_ring},
+               {"V32_KSPLIT=", &t.v32_ksplit}, {"KSPLIT=", &t.ksplit}, {"ROWS32=", &t.rows32},
+               {"XCD_ORDER=", &t.xcd_order}, {"PLAN_FAST_MAX=", &t.plan_fast_max}, {"LDS_RING=", &t.lds_ring},
+               {"SEG_COST=", &t.seg_cost}};
+  for (char** e = environ; e && *e; ++e) {
+    if (strncmp(*e, "KVQ_", 4) != 0) continue;
+    for (const auto& k : known) {
+      const size_t n = strlen(k.name);
+      if (!*k.to && strncmp(*e + 4, k.name, n) == 0) *k.to = *e + 4 + n;
+    }
+  }
+  return t;
+}
+
 // Work units (32-key tiles of one workgroup's streaming) charged per segment for its fixed cost in
 // the stream-K partition, per kernel (KVQ_SEG_COST overrides both). Like the other tuning variables,
 // read at every call.
-int seg_cost_units(bool lds_ring, int v32_key_splits) {
-  const int env = [] {
-    const char* e = getenv("KVQ_SEG_COST");
-    if (!e) return -1;
-    const int v = atoi(e);
-    return v < 0 ? 0 : (v > 64 ? 64 : v);
-  }();
+int seg_cost_units(const Tuning& t, bool lds_ring, int v32_key_splits) {
+  const int env = t.seg_cost ? std::max(0, std::min(64, atoi(t.seg_cost))) : -1;
   // verify_kernel with 2 key splits streams a unit (one 32-key tile of the segment) in half the time, so
   // its fixed cost is more units (c3, 3-slot rings: 12 -> 24 units 68.5 -> 66.1 us, 36 units 67.3, 48
   // units 71.3; 2-slot rings: 16 units 65.1-65.3 us, 24 units 66.1-66.9; with the merge's speculative
@@ -3247,31 +3268,27 @@ int seg_cost_units(bool lds_ring, int v32_key_splits) {
 }
 
 // slots of the attention's shared LDS ring (KVQ_LDS_PREFETCH: 3, 4 or 6)
-int lds_prefetch_depth() {
-  const char* e = getenv("KVQ_LDS_PREFETCH");
-  const int v = e ? atoi(e) : DEFAULT_LDS_PREFETCH;
+int lds_prefetch_depth(const Tuning& t) {
+  const int v = t.lds_prefetch ? atoi(t.lds_prefetch) : DEFAULT_LDS_PREFETCH;
   return v <= 3 ? 3 : (v >= 6 ? 6 : 4);
 }
 
 // slots of verify_kernel's LDS ring (KVQ_V32_RING: 2, 3 or 4; 2 only with two key splits, where it is
 // the fastest on verification batches: 3 or 4 slots took 66.5-67 against 62-64 us on c3)
-int v32_ring_depth() {
-  const char* e = getenv("KVQ_V32_RING");
-  const int v = e ? atoi(e) : DEFAULT_V32_RING;
+int v32_ring_depth(const Tuning& t) {
+  const int v = t.v32_ring ? atoi(t.v32_ring) : DEFAULT_V32_RING;
   return v <= 2 ? 2 : v == 3 ? 3 : 4;
 }
 // verify_kernel's key splits per workgroup (KVQ_V32_KSPLIT: 1 or 2)
-int v32_key_splits() {
-  const char* e = getenv("KVQ_V32_KSPLIT");
-  const int v = e ? atoi(e) : DEFAULT_V32_KSPLIT;
+int v32_key_splits(const Tuning& t) {
+  const int v = t.v32_ksplit ? atoi(t.v32_ksplit) : DEFAULT_V32_KSPLIT;
   return v <= 1 ? 1 : 2;
 }
 
 // Register tiles per wavefront in the attention ring (KVQ_PREFETCH overrides the default; d128 is
 // instantiated for 2, 3, 4, 6, 8 and d64 for 2, 3, 4 -- other values run depth 4).
-int prefetch_depth() {
-  const char* e = getenv("KVQ_PREFETCH");
-  const int v = e ? atoi(e) : DEFAULT_PREFETCH;
+int prefetch_depth(const Tuning& t) {
+  const int v = t.prefetch ? atoi(t.prefetch) : DEFAULT_PREFETCH;
   return v < 2 ? 2 : (v > 8 ? 8 : v);
 }
 
@@ -3800,17 +3817,17 @@ int decode_attention(const void* q, int64_t q_st, int64_t q_sh, const int8_t* k_
   const int rt = (int)std::min<int64_t>(MAX_ROW_TILES, row_tiles);
   // key splits fill up to DEFAULT_KSPLIT wavefronts per row tile, within the workgroup's 4
   // (KVQ_KSPLIT overrides, 1: none)
-  const char* ks_env = getenv("KVQ_KSPLIT");
+  const Tuning tune = read_tuning();
   // Without split buffers nothing is cut across workgroups: as many key splits as the workgroup
   // holds then run each segment
-  const int ks_max = ks_env ? std::max(1, std::min(MAX_ROW_TILES, atoi(ks_env)))
+  const int ks_max = tune.ksplit ? std::max(1, std::min(MAX_ROW_TILES, atoi(tune.ksplit)))
                             : (num_splits == 1 ? MAX_ROW_TILES : DEFAULT_KSPLIT);
   const int ks = std::max(1, std::min(ks_max, MAX_ROW_TILES / rt));
   // more than 32 rows per (request, kv head): the 32-row wavefronts of verify_kernel (KVQ_ROWS32=0: off)
   // (per-32-channel q scales run there for every row count)
   const bool rows32 = q_group == 32 ||
-                      ((int64_t)G * maxq > 32 && !(getenv("KVQ_ROWS32") && atoi(getenv("KVQ_ROWS32")) == 0));
-  const int v32ks = rows32 ? v32_key_splits() : 1;
+                      ((int64_t)G * maxq > 32 && !(tune.rows32 && atoi(tune.rows32) == 0));
+  const int v32ks = rows32 ? v32_key_splits(tune) : 1;
   const int waves = rows32 ? 2 * v32ks : rt * ks;
   if (num_seqs > INT32_MAX - 1 || num_kv_heads > 65535 || (num_q_heads + RED_WAVES - 1) / RED_WAVES > 65535 ||
       (int64_t)G * maxq > INT32_MAX / 2)
@@ -3832,16 +3849,17 @@ int decode_attention(const void* q, int64_t q_st, int64_t q_sh, const int8_t* k_
   a.cut_rows = num_splits > 1 ? (int)std::min<int64_t>(segm_rows, INT32_MAX) : 0;
   a.rt = rows32 ? V32_GROUP_TILES : rt; a.ksplit = rows32 ? v32ks : ks; a.waves = waves;
   a.min_tiles = MIN_SPLIT_TILES * a.ksplit;
-  a.xcd_order = getenv("KVQ_XCD_ORDER") ? atoi(getenv("KVQ_XCD_ORDER")) : 1;
+  a.xcd_order = tune.xcd_order ? atoi(tune.xcd_order) : 1;
   // KVQ_PLAN_FAST_MAX (tests): a lower bound on units sends the plan's scans down the 64-bit path
-  a.plan_fast_max = getenv("KVQ_PLAN_FAST_MAX") ? (int)std::max(1ll, std::min(PLAN_FAST_MAX, atoll(getenv("KVQ_PLAN_FAST_MAX"))))
-                                                : (int)PLAN_FAST_MAX;
+  a.plan_fast_max = tune.plan_fast_max ? (int)std::max(1ll, std::min(PLAN_FAST_MAX, atoll(tune.plan_fast_max)))
+                                       : (int)PLAN_FAST_MAX;
   // row tiles of the same rows without key splits share each K/V tile through an LDS ring
   // (KVQ_LDS_RING=0: off), of lds_prefetch_depth() slots
-  a.lds_ring = (rows32 || (ks == 1 && rt >= 2 && !(getenv("KVQ_LDS_RING") && atoi(getenv("KVQ_LDS_RING")) == 0))) ? 1 : 0;
-  a.seg_cost = seg_cost_units(a.lds_ring != 0, rows32 ? v32ks : 0);
+  a.lds_ring = (rows32 || (ks == 1 && rt >= 2 && !(tune.lds_ring && atoi(tune.lds_ring) == 0))) ? 1 : 0;
+  a.seg_cost = seg_cost_units(tune, a.lds_ring != 0, rows32 ? v32ks : 0);
   // (verify_kernel has 2-slot rings only with key splits: the instantiated depth sizes the LDS below)
-  const int pf = rows32 ? std::max(v32_ring_depth(), v32ks == 2 ? 2 : 3) : a.lds_ring ? lds_prefetch_depth() : prefetch_depth();
+  const int pf = rows32 ? std::max(v32_ring_depth(tune), v32ks == 2 ? 2 : 3)
+                 : a.lds_ring ? lds_prefetch_depth(tune) : prefetch_depth(tune);
   const size_t lds = rows32     ? (size_t)v32_lds_bytes(head_dim, pf, v32ks)
                      : a.lds_ring ? (size_t)pf * 2 * TILE * head_dim
                                   : (size_t)(ks - 1) * rt * MERGE_FIELDS * WAVE * sizeof(float);

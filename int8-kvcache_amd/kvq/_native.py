@@ -9,6 +9,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libkvq_int8.so")
 ABI_VERSION = 12
+ERR_LAUNCH = 2      # KVQ_ERR_LAUNCH
 
 _i64 = ctypes.c_int64
 _ptr = ctypes.c_void_p
@@ -87,4 +88,22 @@ def call(name, *args):
     lib = load()
     rc = getattr(lib, name)(*args)
     if rc != 0:
-        raise NativeError(f"{name}: {lib.kvq_last_error().decode()}")
+        raise error(name)
+
+
+def error(name):
+    """The NativeError of this thread's last failed call."""
+    return NativeError(f"{name}: {load().kvq_last_error().decode()}")
+
+
+def torch_calls():
+    """kvq._torch_calls (csrc/torch_calls.cpp: the operators on torch tensors, host code only) bound to the loaded
+    library, or None where it is not built for this torch: the operators then run their Python checks and the
+    ctypes calls, with the same results."""
+    lib = load()
+    try:
+        from . import _torch_calls
+    except ImportError:
+        return None
+    _torch_calls.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES})
+    return _torch_calls

@@ -2,8 +2,11 @@
 
 Same names, arguments, defaults, environment variables and error behaviour as the reference module
 (kvq/cuda_kernels.py:1-183); the kernels behind it are the gfx950 HIP kernels of libkvq_int8.so,
-reached through its C ABI (include/kvq_int8.h) with ctypes. The library is built in-tree ahead of
-time (int8-kvcache_amd/build.py); ext() loads it and raises if it is missing -- there is no fallback.
+reached through its C ABI (include/kvq_int8.h): from one native function per operator for the plain
+form of its arguments (kvq._torch_calls; eager calls of one layer, host time with and without it: cache write
+18 and 3.6 us, decode attention 30 and 6.9 us, a mixed step 71 and 20 us), otherwise with ctypes after the
+checks below. The library is built in-tree ahead of time (int8-kvcache_amd/build.py); ext() loads it and
+raises if it is missing -- there is no fallback.
 
 Attention on the INT8 cache is split by query length (reference kvq/cuda_kernels.py:1-11):
   * requests with at most SHORT_Q query tokens run the INT8 MFMA kernel (implementation B);
@@ -66,6 +69,9 @@ class _Ext:
 
     def __init__(self):
         _native.load()
+        # the same checks and calls in one native function per operator (None: not built)
+        self.calls = _native.torch_calls()
+        self._prefill = None
 
     # kvq/cuda/int8_kv.cu:554-575
     def quant_cache(self, key, value, kc, vc, slots, ks, vs, kmu):
@@ -268,12 +274,15 @@ class _Ext:
     @property
     def prefill_rows(self):
         """(token, q head) rows per work-list entry of the prefill kernel."""
-        return int(_native.load().kvq_prefill_rows_per_tile())
+        if self._prefill is None:
+            lib = _native.load()
+            self._prefill = int(lib.kvq_prefill_rows_per_tile()), int(lib.kvq_prefill_max_parts())
+        return self._prefill[0]
 
     @property
     def prefill_max_parts(self):
         """Most pieces an entry's keys may be cut into."""
-        return int(_native.load().kvq_prefill_max_parts())
+        return self.prefill_rows and self._prefill[1]
 
 
 def ext():
@@ -288,8 +297,22 @@ def ext():
 def quant_reshape_and_cache(key, value, key_cache, value_cache, slot_mapping, static):
     """Quantize the step's new K/V with the static scales and write them through slot_mapping
     (reference kvq/cuda_kernels.py:42-44)."""
-    ext().quant_cache(key, value, key_cache, value_cache, slot_mapping, static["k_scale"], static["v_scale"],
+    e, args = ext(), (key, value, key_cache, value_cache, slot_mapping, static["k_scale"], static["v_scale"],
                       static["k_mu"])
+    if not _served(e, "quant_cache", *args):
+        e.quant_cache(*args)
+
+
+def _served(e, op, *args):
+    """Whether the native call took the operator (kvq._torch_calls): False where it declined the arguments or the
+    library refused them -- nothing was launched, and the Python path repeats the checks and reports."""
+    calls = getattr(e, "calls", None)
+    if calls is None:
+        return False
+    rc = getattr(calls, op)(*args)
+    if rc == _native.ERR_LAUNCH:
+        raise _native.error(op)
+    return rc == 0
 
 
 def quant_q(q, k_scale, group=None):
@@ -376,9 +399,18 @@ def decode_attention(q, k_cache, v_cache, out, cu_seqlens_q, seq_lens, block_tab
     channels: the B_*_qgroup32 configurations of kvq/int8_ref.py:120-129, an addition to the reference's
     operator API)."""
     so, sm, ss = segm if segm is not None else (None, None, None)
-    ext().int8_decode_attention(q, k_cache, v_cache, out, cu_seqlens_q, seq_lens, block_table, static["k_scale"],
-                                static["v_scale"], softmax_scale, so, sm, ss, max_query_len, SHORT_Q, q_group)
+    e, args = ext(), (q, k_cache, v_cache, out, cu_seqlens_q, seq_lens, block_table, static["k_scale"],
+                      static["v_scale"], softmax_scale, so, sm, ss, max_query_len, SHORT_Q, q_group)
+    if not _served(e, "decode_attention", *args, MAX_SPLITS):
+        e.int8_decode_attention(*args)
     return out
+
+
+def _to_device(arrays, device):
+    """int32 device copies of the numpy arrays, in one transfer (each a view of one buffer, in this order)."""
+    flat = torch.from_numpy(np.concatenate([x.reshape(-1) for x in arrays]).astype(np.int32, copy=False)).to(device)
+    parts = flat.split([x.size for x in arrays])
+    return tuple(p.view(x.shape) for p, x in zip(parts, arrays))
 
 
 @dataclass
@@ -400,7 +432,7 @@ class LongPlan:
 
     def gpu(self, device):
         if self._gpu is None:
-            self._gpu = tuple(torch.from_numpy(a).to(device) for a in (self.src_req, self.src_j, self.block_table))
+            self._gpu = _to_device((self.src_req, self.src_j, self.block_table), device)
         return self._gpu
 
     def tiles(self, group, device, rows=None):
@@ -443,11 +475,7 @@ class LongPlan:
             else:
                 longest, slots = lists[5:]
                 lists = (lists[4], *lists[:4])   # the 16-byte merge entries first
-            flat = torch.from_numpy(np.concatenate([x.astype(np.int32).reshape(-1) for x in lists])).to(device)
-            at, views = 0, []
-            for x in lists:
-                views.append(flat[at:at + x.size].view(x.shape))
-                at += x.size
+            views = _to_device(lists, device)
             pages = self.src_req.shape[0] * self.block_size * hkv * d
             direct = direct_pays(longest, d, pages)
             self._work[(group, hkv, d)] = (PrefillWork(*views, None, None, None, 0, direct) if len(views) == 2 else
@@ -506,10 +534,14 @@ def split_rows(req, row, tiles, hkv, d, fill, max_parts):
     rows balance among themselves: 448 workgroups (2,048 tokens from the start) 62 us whole, 64 cut."""
     if req.shape[0] * hkv >= PREFILL_WHOLE * fill or req.shape[0] == 0:
         return None
-    lo, hi = PREFILL_MIN_PIECE, max(PREFILL_MIN_PIECE, int(tiles.max()))
-    while lo < hi:             # the shortest piece length that fits
+    most, total, budget = int(tiles.max()), int(tiles.sum()), PREFILL_PER_CU * fill // hkv
+    # the shortest piece length e that fits: sum(ceil(t / e)) <= budget, between total / budget and
+    # total / (budget - entries)
+    lo = max(PREFILL_MIN_PIECE, -(-total // max(budget, 1)))
+    hi = max(lo, min(most, -(-total // (budget - req.shape[0])) if budget > req.shape[0] else most))
+    while lo < hi:
         mid = (lo + hi) // 2
-        if int(((tiles + mid - 1) // mid).sum()) * hkv <= PREFILL_PER_CU * fill:
+        if int(((tiles + mid - 1) // mid).sum()) <= budget:
             hi = mid
         else:
             lo = mid + 1
@@ -517,9 +549,9 @@ def split_rows(req, row, tiles, hkv, d, fill, max_parts):
     cut = parts > 1
     pieces = int(parts.sum()) * hkv
     longest = int(((tiles + parts - 1) // parts).max())
-    whole_us = TILE_US * _tile_unit(d) * int(tiles.max())
+    whole_us = TILE_US * _tile_unit(d) * most
     cut_us = (TILE2_US if pieces > fill else TILE_US) * _tile_unit(d) * longest + MERGE_US + PIECE_US * d / 128 * pieces
-    if not cut.any() or cut_us >= whole_us:
+    if longest == most or cut_us >= whole_us:
         return None
     at = np.repeat(np.arange(parts.shape[0]), parts)
     part = np.arange(at.shape[0]) - np.repeat(np.cumsum(parts) - parts, parts)
@@ -583,28 +615,33 @@ def long_attention(q, k_cache, v_cache, out, cu_seqlens_q, seq_lens, block_table
     bit-identical); 0 = the two kernels; unset = 1 or 0, whichever is faster (direct_pays)."""
     bs, h, d = k_cache.shape[1:]
     _check(bs == plan.block_size, f"block size {bs} != plan block size {plan.block_size}")
+    e = ext()
     work = plan.work(q.shape[1] // h, h, d, q.device)
-    tile_req, tile_row = work.tile_req, work.tile_row
-    kt_shape = (plan.src_req.shape[0], bs, h, d)
     if os.environ.get("KVQ_DEBUG_DUMP"):  # the prefill call's metadata, for an offline replay (kvq.debug_dump)
         from . import debug_dump
-        debug_dump.dump_long_call(os.environ["KVQ_DEBUG_DUMP"], q, out, cu_seqlens_q, seq_lens, plan, kt_shape,
-                                  *plan.tiles(q.shape[1] // h, q.device), max_query_len, ext().prefill_rows,
-                                  softmax_scale)
+        debug_dump.dump_long_call(os.environ["KVQ_DEBUG_DUMP"], q, out, cu_seqlens_q, seq_lens, plan,
+                                  (plan.src_req.shape[0], bs, h, d), *plan.tiles(q.shape[1] // h, q.device),
+                                  max_query_len, e.prefill_rows, softmax_scale)
     direct = os.environ.get("KVQ_PREFILL_DIRECT") or ("1" if work.direct else "0")
-    split = work.split(h, ext().prefill_rows, d) if direct in ("0", "1", "fold") else None
-    if direct in ("1", "fold"):
-        # the INT8 pages read directly: no temporary cache ("1": same output bits; "fold": scales folded)
-        ext().int8_prefill_attention(q, k_cache, v_cache, out, cu_seqlens_q, seq_lens, block_table, tile_req,
-                                     tile_row, softmax_scale, static["k_scale"], static["v_scale"], direct == "fold", split)
+    _check(direct in ("0", "1", "fold"), f"KVQ_PREFILL_DIRECT must be 0, 1 or fold, got {direct!r}")
+    ks, vs = static["k_scale"], static["v_scale"]
+    src = plan.gpu(q.device) if direct == "0" else (None, None, None)
+    if _served(e, "long_attention", q, k_cache, v_cache, out, cu_seqlens_q, seq_lens, block_table, ks, vs, softmax_scale,
+               ("0", "1", "fold").index(direct), e.prefill_rows, work.tile_req, work.tile_row, work.tile_piece,
+               work.tile_slot, work.merge, work.slots, *src):
         return out
-    _check(direct == "0", f"KVQ_PREFILL_DIRECT must be 0, 1 or fold, got {direct!r}")
-    src_req, src_j, bt_tmp = plan.gpu(q.device)
-    kt = torch.empty(kt_shape, dtype=q.dtype, device=q.device)
+    split = work.split(h, e.prefill_rows, d)
+    if direct != "0":
+        # the INT8 pages read directly: no temporary cache ("1": same output bits; "fold": scales folded)
+        e.int8_prefill_attention(q, k_cache, v_cache, out, cu_seqlens_q, seq_lens, block_table, work.tile_req,
+                                 work.tile_row, softmax_scale, ks, vs, direct == "fold", split)
+        return out
+    src_req, src_j, bt_tmp = src
+    kt = torch.empty((plan.src_req.shape[0], bs, h, d), dtype=q.dtype, device=q.device)
     vt = torch.empty_like(kt)
-    ext().dequant_pages(k_cache, v_cache, kt, vt, block_table, src_req, src_j, static["k_scale"], static["v_scale"])
-    ext().paged_prefill_attention(q, kt, vt, out, cu_seqlens_q, seq_lens, bt_tmp, tile_req, tile_row, softmax_scale,
-                                  split)
+    e.dequant_pages(k_cache, v_cache, kt, vt, block_table, src_req, src_j, ks, vs)
+    e.paged_prefill_attention(q, kt, vt, out, cu_seqlens_q, seq_lens, bt_tmp, work.tile_req, work.tile_row,
+                              softmax_scale, split)
     return out
 
 

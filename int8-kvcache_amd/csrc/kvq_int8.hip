@@ -54,11 +54,9 @@ constexpr int MIN_SPLIT_TILES = 4;  // shortest split: 4 tiles = 128 keys
 constexpr int DEFAULT_WAVES_PER_CU = 8;
 constexpr int DEFAULT_KSPLIT = 2;     // key splits per row tile: skewed batches (c4) run 9% faster
                                       // than with 4 (2-wavefront workgroups, twice as many); c2 the same
-constexpr int DEFAULT_LDS_PREFETCH = 3;   // shared LDS ring slots (3, 4 and 6 time the same on c3)
 constexpr int DEFAULT_SEG_COST = 8;   // a segment's fixed cost, in tile units: skewed batches (c4's
                                       // lengths; 10 x 32k + 86 x 1 keys) time best at 6-16
-constexpr int DEFAULT_SEG_COST_LDS_RING = 12;  // the same for the LDS-ring kernel (4 row tiles filling
-                                               // one ring): verification batches time best at 12
+constexpr int DEFAULT_SEG_COST_V32 = 12;  // the same for verify_kernel with one key split
 // register ring of the decode kernel: tiles in flight per wavefront (PF - 1 ahead of the one computed).
 // Under full load HBM latency grows with the bytes in flight (~5 us at 2 tiles ahead per wavefront), and
 // every piece of a segment pays it twice at its start (page ids, then K/V): one tile ahead streams as
@@ -542,8 +540,6 @@ struct AttnArgs {
   int num_blocks, lbs, ks_pc, vs_pc;
   int ksplit;         // key splits per workgroup: wavefront (t, k) takes every ksplit-th key tile of row tile t
   int waves;          // rt * ksplit wavefronts per workgroup
-  int lds_ring;       // 1: the workgroup's wavefronts are row tiles of the same rows (ksplit 1, rt >= 2)
-                      // and share each K/V tile through an LDS ring of PF slots (the dynamic LDS)
 };
 static_assert(offsetof(AttnArgs, q) == 64, "the plan's arguments fill the first 64 bytes");
 
@@ -685,7 +681,8 @@ __device__ Plan plan_and_locate(const AttnArgs& a, int lane, int& worker_out, in
     ch = max(ch, (long long)a.min_tiles);
   }
   p.chunk = uniform64(max(ch, 1ll));
-  const int active = (int)min((long long)a.workers, udiv_plan(p.total + p.chunk - 1, p.chunk));
+  // (a full grid, the usual case, needs no division)
+  const int active = p.total > p.chunk * (a.workers - 1) ? a.workers : (int)udiv_plan(p.total + p.chunk - 1, p.chunk);
   int worker = blockIdx.x;
   if (a.xcd_order) {
     const int q = active / NUM_XCDS, rem = active % NUM_XCDS;
@@ -799,7 +796,7 @@ constexpr float ATTN_SLACK = 8.f;  // log2 headroom of the attention's reference
 // wavefront ks = 0 finishes the piece, the segment's `part`-th of `nparts`: a whole segment writes
 // bf16 out, a cut one an fp32 partial. Every wavefront of the workgroup calls this for every piece
 // (inactive ones -- row tiles past the request's rows -- only join the barriers of the merge).
-template <int D, int PF, bool SHARED>
+template <int D, int PF>
 __device__ __forceinline__ void attend_segment(const AttnArgs& a, int seq, int tok, int qlen, int seqlen, int kvh, int row0,
                                                int c_begin, int c_end, int ks, int KS, int rtile, bool active,
                                                int part, int nparts, float* lds, int lane) {
@@ -824,11 +821,8 @@ __device__ __forceinline__ void attend_segment(const AttnArgs& a, int seq, int t
   const int n = lane & 15, g = lane >> 4;
   const int G = a.G;
   const int L = __builtin_amdgcn_readfirstlane(seqlen);
-  // no keys (malformed): nothing is read. A wavefront with no rows reads nothing either -- except
-  // with a shared LDS ring, where it still fetches its share of every tile and keeps the barriers
-  constexpr bool shared = SHARED;  // launched with a.lds_ring set
-  const bool work = L > 0 && active;
-  if (L <= 0 || (!active && !shared)) c_end = c_begin;
+  // no keys (malformed): nothing is read. A wavefront with no rows reads nothing either
+  if (L <= 0 || !active) c_end = c_begin;
   // this wavefront's tiles: c_begin + ks + j * KS, j < nt
   const int nt = c_begin + ks < c_end ? (c_end - c_begin - ks + KS - 1) / KS : 0;
   auto tile = [&](int j) { return c_begin + ks + j * KS; };
@@ -887,130 +881,7 @@ __device__ __forceinline__ void attend_segment(const AttnArgs& a, int seq, int t
     }
   };
 
-  // ---- shared ring: a tile is DMA'd once (global_load_lds_dwordx4, 64 lanes x 16 bytes = RPI rows
-  // per instruction; K rows, then V rows, each row's 16-byte chunks XOR-swizzled by row % CHR so
-  // that the operand reads below spread over the banks); the rt wavefronts issue instruction
-  // rtile + rt u of each tile (u < NIW; past NI an instruction is issued twice -- the same bytes to
-  // the same place) ----
-  constexpr int RB_ = D;                     // bytes per K (or V) row
-  constexpr int CHR = RB_ / 16;              // 16-byte chunks per row
-  constexpr int RPI = WAVE / CHR;            // rows per DMA instruction
-  constexpr int NI = 2 * TILE / RPI;         // DMA instructions per tile (K rows, then V rows)
-  constexpr int SLOT = 2 * TILE * RB_;       // bytes per ring slot
-  uint8_t* lring = reinterpret_cast<uint8_t*>(lds);
-  // lane part of a DMA source address: row lane / CHR of the instruction's RPI rows, chunk lc. The
-  // swizzle row % CHR is (lane / CHR) % CHR whatever the instruction (RPI is a multiple of CHR), so the
-  // offsets are the same for every instruction; the rest of the address is uniform (scalar base).
-  const uint32_t lrow = lane / CHR, lch = 16 * ((lane % CHR) ^ (lrow % CHR));
-  const uint32_t kdo = lrow * (uint32_t)a.k_sn + lch, vdo = lrow * (uint32_t)a.v_sn + lch;
-  auto dma = [&](auto niw_t, int c, int st) {
-    constexpr int NIW = decltype(niw_t)::value;
-    const int n0 = c * TILE, n1 = n0 + 16;
-    const int p0 = page_of(n0);
-    const int p1 = n1 < L ? page_of(n1) : p0;
-    const int o0 = n0 & (bs - 1), o1 = n1 < L ? (n1 & (bs - 1)) : o0;
-#pragma unroll
-    for (int u = 0; u < NIW; ++u) {
-      int i = rtile + a.rt * u;
-      if (i >= NI) i -= NI;
-      const bool isv = i >= NI / 2;
-      const int blk = i % (NI / 2);
-      const bool hi = RPI * blk >= 16;  // rows of one instruction sit in one half of the tile
-      const int p = hi ? p1 : p0, o = (hi ? o1 - 16 : o0) + RPI * blk;
-      const int8_t* sb = isv ? vbase + (int64_t)p * a.v_sb + (int64_t)o * a.v_sn
-                             : kbase + (int64_t)p * a.k_sb + (int64_t)o * a.k_sn;
-      __builtin_amdgcn_global_load_lds((const void*)(sb + (uint64_t)(isv ? vdo : kdo)),
-                                       (__attribute__((address_space(3))) void*)(lring + st * SLOT + (isv ? TILE * RB_ : 0) + 1024 * blk),
-                                       16, 0, 0);
-    }
-  };
-  // this lane's operands of slot st: K as load() would put them in registers (row 16 b + n, logical
-  // chunk (KPL / 16) g + s), and the V^T operands themselves, read with ds_read_b64_tr_b8: within a
-  // 16-lane group, lane 8 h + b receives byte b of the 8-byte chunks addressed by lanes h, h + 2, ...,
-  // h + 14 (element j from lane h + 2 j). So lane (g, h, j = (lane % 16) / 2) addresses key row
-  // 4 g + j (j < 4) or 16 + 4 g + j - 4 -- the key of P operand slot j of lane group g -- at bytes
-  // 16 t + 8 h, and lane (m = 8 h + b, g) receives channel 16 t + m of its 8 keys: channel tile t is
-  // channels 16 t .. 16 t + 15 here (the register path interleaves them, see the epilogue).
-  // Inline assembly, each statement waiting for its own reads: the compiler would otherwise make the
-  // reads wait for every DMA in flight (it cannot tell they read another slot).
-  uint32_t ka0[2][KSTEPS], vta0[VT];  // slot 0's read addresses
-#pragma unroll
-  for (int b = 0; b < 2; ++b)
-#pragma unroll
-    for (int s2 = 0; s2 < KSTEPS; ++s2) {
-      const int row = 16 * b + n;
-      ka0[b][s2] = (uint32_t)(uintptr_t)lring + row * RB_ + 16 * (((KPL / 16) * g + s2) ^ (row % CHR));
-    }
-  {
-    const int j = (lane & 15) >> 1, h = lane & 1;
-    const int row = j < 4 ? 4 * g + j : 16 + 4 * g + j - 4;
-#pragma unroll
-    for (int t = 0; t < VT; ++t)
-      vta0[t] = (uint32_t)(uintptr_t)lring + TILE * RB_ + row * RB_ + 16 * (t ^ (row % CHR)) + 8 * h;
-  }
-  // st_t: the slot, an int or a std::integral_constant (then its offset is the reads' immediate)
-  auto lds_tile = [&](auto st_t, KVTile<D>& r) {
-    constexpr bool CT = !std::is_same_v<decltype(st_t), int>;
-    uint32_t so;
-    if constexpr (CT) so = 0;
-    else so = (uint32_t)(st_t * SLOT);
-    constexpr int IMM = [] {
-      if constexpr (CT) return decltype(st_t)::value * SLOT;
-      else return 0;
-    }();
-    typedef unsigned long long u64;
-    u64 w[VT];
-    if constexpr (D == 128) {
-      asm volatile(
-          "ds_read_b128 %0, %12 offset:%c24\n"
-          "ds_read_b128 %1, %13 offset:%c24\n"
-          "ds_read_b128 %2, %14 offset:%c24\n"
-          "ds_read_b128 %3, %15 offset:%c24\n"
-          "ds_read_b64_tr_b8 %4, %16 offset:%c24\n"
-          "ds_read_b64_tr_b8 %5, %17 offset:%c24\n"
-          "ds_read_b64_tr_b8 %6, %18 offset:%c24\n"
-          "ds_read_b64_tr_b8 %7, %19 offset:%c24\n"
-          "ds_read_b64_tr_b8 %8, %20 offset:%c24\n"
-          "ds_read_b64_tr_b8 %9, %21 offset:%c24\n"
-          "ds_read_b64_tr_b8 %10, %22 offset:%c24\n"
-          "ds_read_b64_tr_b8 %11, %23 offset:%c24\n"
-          "s_waitcnt lgkmcnt(0)"
-          : "=&v"(r.k[0][0]), "=&v"(r.k[0][1]), "=&v"(r.k[1][0]), "=&v"(r.k[1][1]), "=&v"(w[0]), "=&v"(w[1]),
-            "=&v"(w[2]), "=&v"(w[3]), "=&v"(w[4]), "=&v"(w[5]), "=&v"(w[6]), "=&v"(w[7])
-          : "v"(ka0[0][0] + so), "v"(ka0[0][1] + so), "v"(ka0[1][0] + so), "v"(ka0[1][1] + so), "v"(vta0[0] + so),
-            "v"(vta0[1] + so), "v"(vta0[2] + so), "v"(vta0[3] + so), "v"(vta0[4] + so), "v"(vta0[5] + so),
-            "v"(vta0[6] + so), "v"(vta0[7] + so), "i"(IMM)
-          : "memory");
-    } else {
-      asm volatile(
-          "ds_read_b128 %0, %6 offset:%c12\n"
-          "ds_read_b128 %1, %7 offset:%c12\n"
-          "ds_read_b64_tr_b8 %2, %8 offset:%c12\n"
-          "ds_read_b64_tr_b8 %3, %9 offset:%c12\n"
-          "ds_read_b64_tr_b8 %4, %10 offset:%c12\n"
-          "ds_read_b64_tr_b8 %5, %11 offset:%c12\n"
-          "s_waitcnt lgkmcnt(0)"
-          : "=&v"(r.k[0][0]), "=&v"(r.k[1][0]), "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3])
-          : "v"(ka0[0][0] + so), "v"(ka0[1][0] + so), "v"(vta0[0] + so), "v"(vta0[1] + so), "v"(vta0[2] + so),
-            "v"(vta0[3] + so), "i"(IMM)
-          : "memory");
-    }
-    // the V^T operand of channel tile t, two dwords per tile, in r.v's storage
-#pragma unroll
-    for (int t = 0; t < VT; ++t) {
-      r.v[(2 * t) / VW][(2 * t) % VW] = (uint32_t)w[t];
-      r.v[(2 * t + 1) / VW][(2 * t + 1) % VW] = (uint32_t)(w[t] >> 32);
-    }
-  };
-  const int niw = (NI + a.rt - 1) / a.rt;    // DMA instructions per wavefront and tile (uniform)
-  auto with_niw = [&](auto f) {             // f(std::integral_constant<int, NIW>)
-    if (niw == 1) f(std::integral_constant<int, 1>{});
-    else if (niw == 2) f(std::integral_constant<int, 2>{});
-    else if (niw == 3) f(std::integral_constant<int, 3>{});
-    else f(std::integral_constant<int, 4>{});
-  };
-
-  KVTile<D> ring[SHARED ? 1 : PF];  // the register ring (unused with the LDS ring)
+  KVTile<D> ring[PF];  // the register ring
   // ---- q prologue, part 1: the q row and its K scales are requested before the first tiles' K/V, so
   // that waiting for them (vmcnt counts in issue order) does not wait for the tiles, and quantizing q
   // overlaps the tiles' flight ----
@@ -1032,15 +903,8 @@ __device__ __forceinline__ void attend_segment(const AttnArgs& a, int seq, int t
     }
   }
   if (nt > 0) {
-    if constexpr (SHARED) {
-      with_niw([&](auto niw_t) {
 #pragma unroll
-        for (int j = 0; j < PF - 1; ++j) dma(niw_t, tile(min(j, nt - 1)), j);
-      });
-    } else {
-#pragma unroll
-      for (int j = 0; j < PF - 1; ++j) load(ring[j], tile(min(j, nt - 1)));
-    }
+    for (int j = 0; j < PF - 1; ++j) load(ring[j], tile(min(j, nt - 1)));
   }
 
   // ---- q prologue, part 2: fold s_k, one scale per row, quantize (codes of rint(x / s), the rounding
@@ -1092,13 +956,9 @@ __device__ __forceinline__ void attend_segment(const AttnArgs& a, int seq, int t
       for (int s = 0; s < KSTEPS; ++s) z = __builtin_amdgcn_mfma_i32_16x16x64_i8(r.k[b][s], qop[s], z, 0, 0, 0);
       sc[b] = z;
     }
-    // ---- V^T operands: 8x8 byte transpose per channel tile (the LDS ring reads them transposed) ----
+    // ---- V^T operands: 8x8 byte transpose per channel tile ----
     long vop[VT];
-    if constexpr (SHARED) {
-#pragma unroll
-      for (int t = 0; t < VT; ++t)
-        vop[t] = (long)(((uint64_t)r.v[(2 * t + 1) / VW][(2 * t + 1) % VW] << 32) | r.v[(2 * t) / VW][(2 * t) % VW]);
-    } else if constexpr (VW == 2) {
+    if constexpr (VW == 2) {
       static_assert(VT == 8, "head_dim 128: two V dwords per lane and key, 8 channel tiles");
       uint32_t lo[8], hi[8];  // lo[t] = keys j 0..3 of channel tile t, hi[t] = keys j 4..7
       transpose4x4(r.v[0][0], r.v[1][0], r.v[2][0], r.v[3][0], lo[0], lo[1], lo[2], lo[3]);
@@ -1176,53 +1036,7 @@ __device__ __forceinline__ void attend_segment(const AttnArgs& a, int seq, int t
   // prologue. Tiles below full_end have no masked key for any row of the wavefront; the first loop
   // runs whole rounds of them (j < j_full), the second the rest -- both start rounds at j = k * PF,
   // so the ring slot of every tile is a compile-time index. ----
-  if constexpr (SHARED) {
-   if (nt > 0) {
-    // one barrier per tile: this wavefront's DMA of tile j has landed (wait), everyone's has and
-    // everyone is done reading tile j - 1 (barrier), so its slot takes tile j + PF - 1
-    // tiles j < j_full have no masked key for any row of the wavefront: a loop of its own for them,
-    // so that each loop body holds one variant of the tile arithmetic (with both in one body the
-    // accumulators leave it in other registers than they entered, and are copied back every tile)
-    const int full_end = lim_lo > 0 ? lim_lo / TILE : 0;
-    const int j_full = min(nt, full_end > c_begin + ks ? (full_end - c_begin - ks + KS - 1) / KS : 0);
-    with_niw([&](auto niw_t) {
-      constexpr int NIW = decltype(niw_t)::value;
-      KVTile<D> cur;
-      // tile j sits in slot st = j % PF and its DMA goes to slot (j + PF - 1) % PF: ints, or
-      // compile-time constants in the rounds below (the reads' slot offset is then an immediate)
-      auto step = [&](auto masked_t, int j, auto st, auto dst) {
-        wait_vm<(PF - 2) * NIW>();
-        lds_barrier();
-        dma(niw_t, tile(min(j + PF - 1, nt - 1)), (int)dst);
-        if (work) {
-          lds_tile(st, cur);
-          compute(masked_t, cur, tile(j));
-        }
-      };
-      int j = 0;
-      // whole rounds of PF unmasked tiles (a round starts at a multiple of PF: slots 0 .. PF - 1)
-      for (; j + PF <= j_full; j += PF) {
-        auto round_step = [&](auto jj_t) {
-          constexpr int JJ = decltype(jj_t)::value;
-          if constexpr (JJ < PF)
-            step(std::false_type{}, j + JJ, std::integral_constant<int, JJ>{},
-                 std::integral_constant<int, (JJ + PF - 1) % PF>{});
-        };
-        round_step(std::integral_constant<int, 0>{});
-        round_step(std::integral_constant<int, 1>{});
-        round_step(std::integral_constant<int, 2>{});
-        round_step(std::integral_constant<int, 3>{});
-        round_step(std::integral_constant<int, 4>{});
-        round_step(std::integral_constant<int, 5>{});
-        static_assert(PF <= 6, "rounds are written for up to 6 slots");
-      }
-      for (; j < j_full; ++j) step(std::false_type{}, j, j % PF, (j + PF - 1) % PF);
-      for (; j < nt; ++j) step(std::true_type{}, j, j % PF, (j + PF - 1) % PF);
-    });
-    wait_vm<0>();   // the ring is empty and read before the next piece refills it
-    lds_barrier();
-   }
-  } else if (nt > 0) {
+  if (nt > 0) {
     const int full_end = lim_lo > 0 ? lim_lo / TILE : 0;
     const int j_full = min(nt, full_end > c_begin + ks ? (full_end - c_begin - ks + KS - 1) / KS : 0);
     int j0 = 0;
@@ -1244,8 +1058,7 @@ __device__ __forceinline__ void attend_segment(const AttnArgs& a, int seq, int t
     }
   }
 
-  // ---- epilogue: lane (n, g) holds channels (D/4) g + (D/16) i + t of row n in acc[t][i] (register
-  // path), or channels 16 t + 4 g + i (LDS ring path) ----
+  // ---- epilogue: lane (n, g) holds channels (D/4) g + (D/16) i + t of row n in acc[t][i] ----
   l = group4_sum(l);
   if (KS > 1) {
     // key-split merge (the formula of split_reduce_kernel): wavefronts k >= 1 publish (m, l, acc),
@@ -1289,36 +1102,6 @@ __device__ __forceinline__ void attend_segment(const AttnArgs& a, int seq, int t
   constexpr int OPL = D / 4;
   const int head = kvh * G + rh;
   const int qt = tok + rtok;
-  if constexpr (SHARED) {
-    float vsc[VT][4];
-#pragma unroll
-    for (int t = 0; t < VT; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) vsc[t][i] = a.vs_pc ? a.vs[kvh * D + 16 * t + 4 * g + i] : a.vs[kvh];
-    if (nparts == 1) {
-      if (a.max_splits > 1 && qt < a.cut_rows && g == 0)
-        a.segm_sum[(int64_t)qt * a.seg_st + (int64_t)head * a.seg_sh] = -1.f;
-      const float inv = 1.f / __builtin_fmaxf(l, 1e-30f);
-      uint16_t* orow = a.out + (int64_t)qt * a.o_st + (int64_t)head * a.o_sh + 4 * g;
-#pragma unroll
-      for (int t = 0; t < VT; ++t)
-        *reinterpret_cast<u32x2*>(orow + 16 * t) =
-            u32x2{pack_bf16x2((acc[t][0] * inv) * vsc[t][0], (acc[t][1] * inv) * vsc[t][1]),
-                  pack_bf16x2((acc[t][2] * inv) * vsc[t][2], (acc[t][3] * inv) * vsc[t][3])};
-    } else {
-      const int64_t sidx = (int64_t)qt * a.seg_st + (int64_t)head * a.seg_sh + part;
-      if (g == 0) {
-        a.segm_max[sidx] = m;
-        a.segm_sum[sidx] = part == nparts - 1 ? -2.f - l : l;
-      }
-      float* sp = a.segm_out + sidx * D + 4 * g;
-#pragma unroll
-      for (int t = 0; t < VT; ++t)
-        *reinterpret_cast<float4*>(sp + 16 * t) =
-            float4{acc[t][0] * vsc[t][0], acc[t][1] * vsc[t][1], acc[t][2] * vsc[t][2], acc[t][3] * vsc[t][3]};
-    }
-    return;
-  }
   float vsc[OPL];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -1360,12 +1143,12 @@ __device__ __forceinline__ void attend_segment(const AttnArgs& a, int seq, int t
 
 // Stream-K attention: workgroup w walks units [w * chunk, (w + 1) * chunk) of the batch (the plan of
 // plan_and_locate), segment by segment. Its rt * ks wavefronts split each piece: rt consecutive
-// 16-row tiles (they stream the same K/V tiles at the same time -- the second and later reads hit
-// L1/L2), each over ks interleaved sets of key tiles merged through LDS at the end of the piece.
+// 16-row tiles (more than one only with KVQ_ROWS32=0: they stream the same K/V tiles at the same time, the
+// second and later reads hit L1/L2), each over ks interleaved sets of key tiles merged through LDS at the end of the piece.
 // Decode rows (one row tile) use 2 key splits, so a workgroup covers 2x the keys of one wavefront and
 // a long request's (kv head) is cut across workgroups half as often. Pieces too short for every key
 // split to stream COOP_TILES tiles are not split: the key splits take them in turn, each alone.
-template <int D, int PF, bool SHARED = false>
+template <int D, int PF>
 __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
   // the wavefront index is uniform across the wavefront: keep it (and all row bookkeeping) scalar
   const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
@@ -1401,11 +1184,11 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
     if (c1 <= c0) {
       // fixed-cost units only: nothing to stream here (uniform across the workgroup)
     } else if (a.ksplit > 1 && c1 - c0 >= a.ksplit * COOP_TILES) {
-      attend_segment<D, PF, SHARED>(a, r, w.tok, w.qlen, w.len, kvh, row0, c0, c1, kspl, a.ksplit, rtile, row0 < w.qlen * a.G,
+      attend_segment<D, PF>(a, r, w.tok, w.qlen, w.len, kvh, row0, c0, c1, kspl, a.ksplit, rtile, row0 < w.qlen * a.G,
                             (int)(worker - first), (int)(last - first + 1), merge_lds, lane);
     } else {
       if (solo % a.ksplit == kspl)
-        attend_segment<D, PF, SHARED>(a, r, w.tok, w.qlen, w.len, kvh, row0, c0, c1, 0, 1, rtile, row0 < w.qlen * a.G,
+        attend_segment<D, PF>(a, r, w.tok, w.qlen, w.len, kvh, row0, c0, c1, 0, 1, rtile, row0 < w.qlen * a.G,
                               (int)(worker - first), (int)(last - first + 1), merge_lds, lane);
       ++solo;
     }
@@ -1425,7 +1208,7 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// Verification-shape attention: more than 32 (token, q head) rows per (request, kv head), e.g. 8
+// Verification-shape attention: more than 16 (token, q head) rows per (request, kv head), e.g. 8
 // speculative tokens x 7 q heads = 56 rows. A workgroup of 2 x KS wavefronts takes a piece of one
 // (request, kv head, group of 64 rows): row wavefront rw owns rows row0 = 32 rw .. 32 rw + 31 of the
 // group, key split kw streams the piece's tiles kw, kw + KS, ...; the two row wavefronts of a key split
@@ -3228,17 +3011,17 @@ int log2i(int64_t x) {
 // The attention's tuning variables, read at every call in one pass over the environment (a getenv each is a pass
 // each: about 2 us of a call's host time together).
 struct Tuning {
-  const char *prefetch = nullptr, *lds_prefetch = nullptr, *v32_ring = nullptr, *v32_ksplit = nullptr, *ksplit = nullptr,
-             *rows32 = nullptr, *xcd_order = nullptr, *plan_fast_max = nullptr, *lds_ring = nullptr, *seg_cost = nullptr;
+  const char *prefetch = nullptr, *v32_ring = nullptr, *v32_ksplit = nullptr, *ksplit = nullptr,
+             *rows32 = nullptr, *xcd_order = nullptr, *plan_fast_max = nullptr, *seg_cost = nullptr;
 };
 Tuning read_tuning() {
   Tuning t;
   const struct {
     const char* name;
     const char** to;
-  } known[] = {{"PREFETCH=", &t.prefetch}, {"LDS_PREFETCH=", &t.lds_prefetch}, {"V32_RING=", &t.v32_ring},
+  } known[] = {{"PREFETCH=", &t.prefetch}, {"V32_RING=", &t.v32_ring},
                {"V32_KSPLIT=", &t.v32_ksplit}, {"KSPLIT=", &t.ksplit}, {"ROWS32=", &t.rows32},
-               {"XCD_ORDER=", &t.xcd_order}, {"PLAN_FAST_MAX=", &t.plan_fast_max}, {"LDS_RING=", &t.lds_ring},
+               {"XCD_ORDER=", &t.xcd_order}, {"PLAN_FAST_MAX=", &t.plan_fast_max},
                {"SEG_COST=", &t.seg_cost}};
   for (char** e = environ; e && *e; ++e) {
     if (strncmp(*e, "KVQ_", 4) != 0) continue;
@@ -3253,7 +3036,7 @@ Tuning read_tuning() {
 // Work units (32-key tiles of one workgroup's streaming) charged per segment for its fixed cost in
 // the stream-K partition, per kernel (KVQ_SEG_COST overrides both). Like the other tuning variables,
 // read at every call.
-int seg_cost_units(const Tuning& t, bool lds_ring, int v32_key_splits) {
+int seg_cost_units(const Tuning& t, int v32_key_splits) {
   const int env = t.seg_cost ? std::max(0, std::min(64, atoi(t.seg_cost))) : -1;
   // verify_kernel with 2 key splits streams a unit (one 32-key tile of the segment) in half the time, so
   // its fixed cost is more units (c3, 3-slot rings: 12 -> 24 units 68.5 -> 66.1 us, 36 units 67.3, 48
@@ -3264,13 +3047,7 @@ int seg_cost_units(const Tuning& t, bool lds_ring, int v32_key_splits) {
   // the plan)
   if (env >= 0) return env;
   if (v32_key_splits == 2) return DEFAULT_SEG_COST_V32_KS2;
-  return lds_ring ? DEFAULT_SEG_COST_LDS_RING : DEFAULT_SEG_COST;
-}
-
-// slots of the attention's shared LDS ring (KVQ_LDS_PREFETCH: 3, 4 or 6)
-int lds_prefetch_depth(const Tuning& t) {
-  const int v = t.lds_prefetch ? atoi(t.lds_prefetch) : DEFAULT_LDS_PREFETCH;
-  return v <= 3 ? 3 : (v >= 6 ? 6 : 4);
+  return v32_key_splits ? DEFAULT_SEG_COST_V32 : DEFAULT_SEG_COST;
 }
 
 // slots of verify_kernel's LDS ring (KVQ_V32_RING: 2, 3 or 4; 2 only with two key splits, where it is
@@ -3823,10 +3600,15 @@ int decode_attention(const void* q, int64_t q_st, int64_t q_sh, const int8_t* k_
   const int ks_max = tune.ksplit ? std::max(1, std::min(MAX_ROW_TILES, atoi(tune.ksplit)))
                             : (num_splits == 1 ? MAX_ROW_TILES : DEFAULT_KSPLIT);
   const int ks = std::max(1, std::min(ks_max, MAX_ROW_TILES / rt));
-  // more than 32 rows per (request, kv head): the 32-row wavefronts of verify_kernel (KVQ_ROWS32=0: off)
+  // more than one 16-row tile per (request, kv head): the 32-row wavefronts of verify_kernel, whose row
+  // wavefronts share each K/V tile through LDS (KVQ_ROWS32=0: off). Two row tiles of attn_kernel each stream
+  // and transpose every tile themselves; graph, same box, 28 / 4 heads: 24 requests x 4 tokens (28 rows)
+  // 36.7 -> 25.3 us, 64 x 4 66.9 -> 54.2, 24 x 3 (21 rows) 30.4 -> 23.7, 16 x 5 of 32 / 8 heads (20 rows) 41.0 ->
+  // 28.9; 2 requests x 4 17.7 and 17.9. One row tile (decode) stays with attn_kernel: 96 ragged requests 101
+  // against 114 us there, 1 x 4,096 keys 14.9 against 16.8.
   // (per-32-channel q scales run there for every row count)
   const bool rows32 = q_group == 32 ||
-                      ((int64_t)G * maxq > 32 && !(tune.rows32 && atoi(tune.rows32) == 0));
+                      ((int64_t)G * maxq > 16 && !(tune.rows32 && atoi(tune.rows32) == 0));
   const int v32ks = rows32 ? v32_key_splits(tune) : 1;
   const int waves = rows32 ? 2 * v32ks : rt * ks;
   if (num_seqs > INT32_MAX - 1 || num_kv_heads > 65535 || (num_q_heads + RED_WAVES - 1) / RED_WAVES > 65535 ||
@@ -3853,16 +3635,11 @@ int decode_attention(const void* q, int64_t q_st, int64_t q_sh, const int8_t* k_
   // KVQ_PLAN_FAST_MAX (tests): a lower bound on units sends the plan's scans down the 64-bit path
   a.plan_fast_max = tune.plan_fast_max ? (int)std::max(1ll, std::min(PLAN_FAST_MAX, atoll(tune.plan_fast_max)))
                                        : (int)PLAN_FAST_MAX;
-  // row tiles of the same rows without key splits share each K/V tile through an LDS ring
-  // (KVQ_LDS_RING=0: off), of lds_prefetch_depth() slots
-  a.lds_ring = (rows32 || (ks == 1 && rt >= 2 && !(tune.lds_ring && atoi(tune.lds_ring) == 0))) ? 1 : 0;
-  a.seg_cost = seg_cost_units(tune, a.lds_ring != 0, rows32 ? v32ks : 0);
+  a.seg_cost = seg_cost_units(tune, rows32 ? v32ks : 0);
   // (verify_kernel has 2-slot rings only with key splits: the instantiated depth sizes the LDS below)
-  const int pf = rows32 ? std::max(v32_ring_depth(tune), v32ks == 2 ? 2 : 3)
-                 : a.lds_ring ? lds_prefetch_depth(tune) : prefetch_depth(tune);
-  const size_t lds = rows32     ? (size_t)v32_lds_bytes(head_dim, pf, v32ks)
-                     : a.lds_ring ? (size_t)pf * 2 * TILE * head_dim
-                                  : (size_t)(ks - 1) * rt * MERGE_FIELDS * WAVE * sizeof(float);
+  const int pf = rows32 ? std::max(v32_ring_depth(tune), v32ks == 2 ? 2 : 3) : prefetch_depth(tune);
+  const size_t lds = rows32 ? (size_t)v32_lds_bytes(head_dim, pf, v32ks)
+                            : (size_t)(ks - 1) * rt * MERGE_FIELDS * WAVE * sizeof(float);
   void (*kern)(AttnArgs);
   if (rows32) {
     auto pick = [&](auto qg_t) -> void (*)(AttnArgs) {
@@ -3877,9 +3654,6 @@ int decode_attention(const void* q, int64_t q_st, int64_t q_sh, const int8_t* k_
       return pf == 3 ? verify_kernel<64, 3, QG, 1> : verify_kernel<64, 4, QG, 1>;
     };
     kern = q_group == 32 ? pick(std::integral_constant<int, 32>{}) : pick(std::integral_constant<int, 0>{});
-  } else if (a.lds_ring) {
-    if (head_dim == 128) kern = pf == 3 ? attn_kernel<128, 3, true> : pf == 6 ? attn_kernel<128, 6, true> : attn_kernel<128, 4, true>;
-    else kern = pf == 3 ? attn_kernel<64, 3, true> : pf == 6 ? attn_kernel<64, 6, true> : attn_kernel<64, 4, true>;
   } else if (head_dim == 128) {
     kern = pf == 2 ? attn_kernel<128, 2> : pf == 3 ? attn_kernel<128, 3> : pf == 6 ? attn_kernel<128, 6>
          : pf == 8 ? attn_kernel<128, 8> : attn_kernel<128, 4>;

@@ -538,6 +538,7 @@ struct AttnArgs {
   int64_t q_st, q_sh, o_st, o_sh, k_sb, k_sn, k_sh, v_sb, v_sn, v_sh, seg_st, seg_sh, bt_stride;
   float sm_log2;      // softmax_scale * log2(e)
   int num_blocks, lbs, ks_pc, vs_pc;
+  unsigned g_inv;     // ceil(2^32 / G) where R / G = umulhi(R, g_inv) for every row index R of the call, else 0
   int ksplit;         // key splits per workgroup: wavefront (t, k) takes every ksplit-th key tile of row tile t
   int waves;          // rt * ksplit wavefronts per workgroup
 };
@@ -547,6 +548,37 @@ __device__ __forceinline__ long long uniform64(long long x) {
   const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)(x & 0xffffffffll));
   const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)((unsigned long long)x >> 32));
   return (long long)(((unsigned long long)hi << 32) | lo);
+}
+
+// The kernel's arguments read anew from the kernel argument segment (scalar loads, cache hits once `touch_args`
+// has run). A kernel that takes AttnArgs alone calls it at the start of a phase: the fields of the other phases
+// then hold no scalar registers through it (kept from one load at entry, they were spilled to vector lanes and
+// read back, several hundred instructions per piece).
+__device__ __forceinline__ const AttnArgs& fresh_args() {
+  auto* p = (const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const AttnArgs*)p;
+}
+// Bring every 64-byte line of the arguments into the scalar cache at entry, with the plan's own first load: met
+// one by one later, each is a memory round trip on the way to the first tile.
+__device__ __forceinline__ void touch_args() {
+  const __attribute__((address_space(4))) int* p = (const __attribute__((address_space(4))) int*)__builtin_amdgcn_kernarg_segment_ptr();
+  static_assert(sizeof(AttnArgs) > 256 && sizeof(AttnArgs) <= 320, "five lines");
+  const int x1 = p[16], x2 = p[32], x3 = p[48], x4 = p[64];
+  asm volatile("" ::"s"(x1), "s"(x2), "s"(x3), "s"(x4));
+}
+// x / rt for the 1 .. 4 row tiles of a group
+__device__ __forceinline__ int div_row_tiles(int x, int rt) { return rt == 1 ? x : rt == 4 ? x >> 2 : x / rt; }
+// floor(x / d) for 0 <= x < 2^31 and 0 < d <= 2^30 with a quotient below 2^20: rd = 1 / d to an ulp, so the
+// product is off by less than one
+__device__ __forceinline__ int div_small(int x, int d, float rd) {
+  int q = (int)((float)x * rd);
+  const int r = x - q * d;
+  return __builtin_amdgcn_readfirstlane(r < 0 ? q - 1 : r >= d ? q + 1 : q);
+}
+// R / G for a row index: by multiplication with ceil(2^32 / G) where the host found that exact (a.g_inv != 0)
+__device__ __forceinline__ int div_group(const AttnArgs& a, int R) {
+  return a.G == 1 ? R : a.g_inv ? (int)__umulhi((unsigned)R, a.g_inv) : R / a.G;
 }
 
 // What one request asks of the kernel: its 32-key tiles (at least one) and row groups (of `waves`
@@ -562,7 +594,7 @@ __device__ __forceinline__ ReqWork req_work(const AttnArgs& a, int r) {
   if (w.qlen <= 0 || w.qlen > a.qmax) return w;
   w.ntiles = max(1, (w.len + TILE - 1) / TILE);
   const int rt = (w.qlen * a.G + 15) / 16;
-  w.rgroups = (rt + a.rt - 1) / a.rt;
+  w.rgroups = div_row_tiles(rt + a.rt - 1, a.rt);
   return w;
 }
 // Whether the request's segments may be cut across workgroups: split buffers exist and hold rows for
@@ -677,7 +709,7 @@ __device__ Plan plan_and_locate(const AttnArgs& a, int lane, int& worker_out, in
   p.total = tot;
   long long ch = udiv_plan(p.total + a.workers - 1, a.workers);
   if (nmax > 0) {
-    ch = max(ch, (long long)((nmax + a.max_splits - 2) / (a.max_splits - 1)));
+    if (ch * (a.max_splits - 1) < nmax) ch = (nmax + a.max_splits - 2) / (a.max_splits - 1);
     ch = max(ch, (long long)a.min_tiles);
   }
   p.chunk = uniform64(max(ch, 1ll));
@@ -718,13 +750,74 @@ __device__ Plan plan_and_locate(const AttnArgs& a, int lane, int& worker_out, in
       f.qlen = __builtin_amdgcn_readlane(w.qlen, idx);
       f.len = __builtin_amdgcn_readlane(w.len, idx);
       f.ntiles = max(1, (f.len + TILE - 1) / TILE);
-      f.rgroups = ((f.qlen * a.G + 15) / 16 + a.rt - 1) / a.rt;
+      f.rgroups = div_row_tiles((f.qlen * a.G + 15) / 16 + a.rt - 1, a.rt);
       w_out = f;
       break;
     }
     base += ctot;
   }
   return p;
+}
+
+// The pieces of this workgroup's worker, in order: f(r, w, kvh, rg, c0, c1, part, nparts) for tiles [c0, c1) of row
+// group rg of kv head kvh of request r (work w), piece `part` of the segment's nparts. Worker w takes units
+// [w chunk, (w + 1) chunk); a segment's first seg_cost units stand for its fixed cost, the rest for its tiles:
+// pieces are the workers' shares of the tile units (a worker holding only fixed-cost units has no piece, and the
+// pieces are numbered from the worker holding the first tile). A segment that may not be cut is run whole by the
+// worker where it starts, one piece. Positions are counted from the worker's first unit, so that a piece's number
+// needs a small quotient by the chunk and only where the segment reaches beyond this worker. The front of a
+// kernel, entry to first page id, took 3.0 us with 64-bit positions and divisions, 2.4 of them arithmetic; with
+// this and fresh_args, in graphs on one box: 1 x 4,096 keys 14.9 -> 14.3 us, 8 x 2k 17.9 -> 17.3, 24 x 4-token
+// verification 25.7 -> 24.0, 64 x 8 57.9 -> 56.8, c4's ragged decode rows 104.6 -> 103.4, 128 x 32k unchanged.
+template <typename F>
+__device__ __forceinline__ void walk_pieces(const AttnArgs& a, int lane, F&& f) {
+  int worker, r;
+  long long rstart;
+  ReqWork w;
+  const Plan pl = plan_and_locate(a, lane, worker, r, rstart, w);
+  if (r >= a.num_seqs) return;
+  const long long w0 = (long long)worker * pl.chunk;
+  const long long len = min(pl.chunk, pl.total - w0);    // this worker's units
+  const int chunk = (int)min(pl.chunk, 1ll << 30);       // (a longer chunk holds more than any one segment)
+  const float rchunk = 1.f / (float)chunk;
+  const int fc = a.seg_cost;
+  int seglen = seg_units(a, w);
+  const int seg = (int)udiv_plan(w0 - rstart, seglen);
+  long long at = rstart + (long long)seg * seglen - w0;  // the segment's first unit, from w0
+  int kvh = seg, rg = 0;
+  if (w.rgroups > 1) {
+    kvh = seg / w.rgroups;
+    rg = seg - kvh * w.rgroups;
+  }
+  bool whole = !cuttable(a, w);
+  for (;;) {
+    const int off = (int)max(-at, 0ll), upto = (int)min((long long)seglen, len - at);
+    const int c0 = whole ? 0 : max(off - fc, 0);
+    const int c1 = whole ? (off == 0 ? w.ntiles : 0) : max(upto - fc, 0);
+    if (c1 > c0) {  // (otherwise fixed-cost units only: nothing to stream here, uniform across the workgroup)
+      int part = 0, after = 0;   // workers with tiles of the segment before and after this one
+      if (!whole) {
+        if (off > fc) part = div_small(off - fc + chunk - 1, chunk, rchunk);
+        const long long z = at + seglen - 1;
+        if (z >= pl.chunk) after = pl.chunk > chunk ? 1 : div_small((int)z, chunk, rchunk);
+      }
+      f(r, w, kvh, rg, c0, c1, part, part + after + 1);
+    }
+    at += seglen;
+    if (at >= len) return;
+    if (++rg == w.rgroups) {
+      rg = 0;
+      if (++kvh == a.hkv) {  // on to the next request with work
+        kvh = 0;
+        do {
+          if (++r >= a.num_seqs) return;
+          w = req_work(a, r);
+        } while (w.ntiles == 0);
+        seglen = seg_units(a, w);
+        whole = !cuttable(a, w);
+      }
+    }
+  }
 }
 
 // K/V pages are streamed exactly once per launch: the non-temporal hint keeps them from evicting
@@ -784,11 +877,53 @@ constexpr int MERGE_SLOTS = MAX_ROW_TILES - 1;
 // Shortest piece split across a workgroup's key splits, in tiles per key split: shorter pieces go
 // whole to one key split in turn (no barrier, no merge). c4's decode rows: 2, 3, 4 all 117.8-118.0 us,
 // 6 119.0, 8 119.3, 16 121.9 us.
-#ifndef KVQ_COOP_TILES
-#define KVQ_COOP_TILES 4
-#endif
-constexpr int COOP_TILES = KVQ_COOP_TILES;
+constexpr int COOP_TILES = 4;
 constexpr float ATTN_SLACK = 8.f;  // log2 headroom of the attention's reference maximum
+
+// The end of a piece: lane group g writes channels (D/4) g .. + D/4 - 1 of its row (token qt, q head `head`) -- bf16
+// out of a whole segment, or the fp32 partial of a cut one. acc[t][i] is channel (D/4) g + (D/16) i + t.
+template <int D>
+__device__ __forceinline__ void finish_segment(const AttnArgs& a, int kvh, int qt, int head, int g, float m, float l,
+                                               const float (&acc)[D / 16][4], int part, int nparts) {
+  constexpr int OPL = D / 4, VT = D / 16;
+  float vsc[OPL];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int t = 0; t < VT; ++t) vsc[VT * i + t] = a.vs_pc ? a.vs[kvh * D + OPL * g + VT * i + t] : a.vs[kvh];
+  if (nparts == 1) {
+    // a row that is not cut tells the merge kernel so: -1 in its piece-0 denominator slot
+    if (a.max_splits > 1 && qt < a.cut_rows && g == 0)
+      a.segm_sum[(int64_t)qt * a.seg_st + (int64_t)head * a.seg_sh] = -1.f;
+    const float inv = 1.f / __builtin_fmaxf(l, 1e-30f);
+    uint32_t o[OPL / 2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int t = 0; t < VT; t += 2)
+        o[(VT * i + t) / 2] = pack_bf16x2((acc[t][i] * inv) * vsc[VT * i + t], (acc[t + 1][i] * inv) * vsc[VT * i + t + 1]);
+    u32x4* op = reinterpret_cast<u32x4*>(a.out + (int64_t)qt * a.o_st + (int64_t)head * a.o_sh + OPL * g);
+#pragma unroll
+    for (int u = 0; u < OPL / 8; ++u) op[u] = u32x4{o[4 * u], o[4 * u + 1], o[4 * u + 2], o[4 * u + 3]};
+  } else {
+    const int64_t sidx = (int64_t)qt * a.seg_st + (int64_t)head * a.seg_sh + part;
+    if (g == 0) {
+      a.segm_max[sidx] = m;
+      a.segm_sum[sidx] = part == nparts - 1 ? -2.f - l : l;  // the last piece is marked (l >= 0)
+    }
+    float* sp = a.segm_out + sidx * D + OPL * g;
+#pragma unroll
+    for (int u = 0; u < OPL / 4; ++u) {
+      float4 w;
+      const int c0 = 4 * u;
+      w.x = acc[(c0 + 0) % VT][(c0 + 0) / VT] * vsc[c0 + 0];
+      w.y = acc[(c0 + 1) % VT][(c0 + 1) / VT] * vsc[c0 + 1];
+      w.z = acc[(c0 + 2) % VT][(c0 + 2) / VT] * vsc[c0 + 2];
+      w.w = acc[(c0 + 3) % VT][(c0 + 3) / VT] * vsc[c0 + 3];
+      reinterpret_cast<float4*>(sp)[u] = w;
+    }
+  }
+}
 
 // One wavefront's share of one piece of a segment: its 16-row tile (rows row0..row0+15 of the
 // (token, q head) rows of kv head kvh) over the key tiles c_begin + ks, c_begin + ks + KS, ... below
@@ -797,9 +932,11 @@ constexpr float ATTN_SLACK = 8.f;  // log2 headroom of the attention's reference
 // bf16 out, a cut one an fp32 partial. Every wavefront of the workgroup calls this for every piece
 // (inactive ones -- row tiles past the request's rows -- only join the barriers of the merge).
 template <int D, int PF>
-__device__ __forceinline__ void attend_segment(const AttnArgs& a, int seq, int tok, int qlen, int seqlen, int kvh, int row0,
-                                               int c_begin, int c_end, int ks, int KS, int rtile, bool active,
-                                               int part, int nparts, float* lds, int lane) {
+__device__ __forceinline__ void attend_segment(int seq, int tok, int qlen, int seqlen, int kvh, int row0, int c_begin,
+                                               int c_end, int ks, int KS, int rtile, int part, int nparts, float* lds,
+                                               int lane) {
+  const AttnArgs& a = fresh_args();
+  const bool active = row0 < qlen * a.G;
   constexpr int KPL = D / 4;        // K bytes per lane and key
   constexpr int KSTEPS = D / 64;    // x64 MFMAs per 16-key block
   constexpr int VT = D / 16;        // PV channel tiles = V bytes per lane and key
@@ -830,11 +967,11 @@ __device__ __forceinline__ void attend_segment(const AttnArgs& a, int seq, int t
   const int bs = 1 << a.lbs;
 
   i32x4 qop[KSTEPS];
-  const int R = row0 + n, rtok = R / G, rh = R % G;
+  const int R = row0 + n, rtok = div_group(a, R), rh = R - rtok * G;
   float rs;
   int lim;
   // every row of this wavefront sees at least keys < lim_lo
-  const int lim_lo = L - qlen + 1 + row0 / G;
+  const int lim_lo = L - qlen + 1 + __builtin_amdgcn_readfirstlane(div_group(a, row0));
 
   float m = -1e30f, l = 0.f, acc[VT][4];
 #pragma unroll
@@ -1099,48 +1236,8 @@ __device__ __forceinline__ void attend_segment(const AttnArgs& a, int seq, int t
     __syncthreads();  // the slots are rewritten by the next piece
   }
   if (ks > 0 || !active || rtok >= qlen) return;
-  constexpr int OPL = D / 4;
-  const int head = kvh * G + rh;
-  const int qt = tok + rtok;
-  float vsc[OPL];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int t = 0; t < VT; ++t) vsc[VT * i + t] = a.vs_pc ? a.vs[kvh * D + OPL * g + VT * i + t] : a.vs[kvh];
-  if (nparts == 1) {
-    // a row that is not cut tells the merge kernel so: -1 in its piece-0 denominator slot
-    if (a.max_splits > 1 && qt < a.cut_rows && g == 0)
-      a.segm_sum[(int64_t)qt * a.seg_st + (int64_t)head * a.seg_sh] = -1.f;
-    const float inv = 1.f / __builtin_fmaxf(l, 1e-30f);
-    uint32_t o[OPL / 2];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int t = 0; t < VT; t += 2)
-        o[(VT * i + t) / 2] = pack_bf16x2((acc[t][i] * inv) * vsc[VT * i + t], (acc[t + 1][i] * inv) * vsc[VT * i + t + 1]);
-    u32x4* op = reinterpret_cast<u32x4*>(a.out + (int64_t)qt * a.o_st + (int64_t)head * a.o_sh + OPL * g);
-#pragma unroll
-    for (int u = 0; u < OPL / 8; ++u) op[u] = u32x4{o[4 * u], o[4 * u + 1], o[4 * u + 2], o[4 * u + 3]};
-  } else {
-    const int64_t sidx = (int64_t)qt * a.seg_st + (int64_t)head * a.seg_sh + part;
-    if (g == 0) {
-      a.segm_max[sidx] = m;
-      a.segm_sum[sidx] = part == nparts - 1 ? -2.f - l : l;  // the last piece is marked (l >= 0)
-    }
-    float* sp = a.segm_out + sidx * D + OPL * g;
-#pragma unroll
-    for (int u = 0; u < OPL / 4; ++u) {
-      float4 w;
-      const int c0 = 4 * u;
-      w.x = acc[(c0 + 0) % VT][(c0 + 0) / VT] * vsc[c0 + 0];
-      w.y = acc[(c0 + 1) % VT][(c0 + 1) / VT] * vsc[c0 + 1];
-      w.z = acc[(c0 + 2) % VT][(c0 + 2) / VT] * vsc[c0 + 2];
-      w.w = acc[(c0 + 3) % VT][(c0 + 3) / VT] * vsc[c0 + 3];
-      reinterpret_cast<float4*>(sp)[u] = w;
-    }
-  }
+  finish_segment<D>(fresh_args(), kvh, tok + rtok, kvh * G + rh, g, m, l, acc, part, nparts);
 }
-
 // Stream-K attention: workgroup w walks units [w * chunk, (w + 1) * chunk) of the batch (the plan of
 // plan_and_locate), segment by segment. Its rt * ks wavefronts split each piece: rt consecutive
 // 16-row tiles (more than one only with KVQ_ROWS32=0: they stream the same K/V tiles at the same time, the
@@ -1150,61 +1247,25 @@ __device__ __forceinline__ void attend_segment(const AttnArgs& a, int seq, int t
 // split to stream COOP_TILES tiles are not split: the key splits take them in turn, each alone.
 template <int D, int PF>
 __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
+  touch_args();
   // the wavefront index is uniform across the wavefront: keep it (and all row bookkeeping) scalar
   const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-  const int rtile = wave % a.rt, kspl = wave / a.rt;  // row tile and key split of this wavefront
+  // row tile and key split of this wavefront
+  const int rt = a.rt, ksplit = a.ksplit, kspl = div_row_tiles(wave, rt), rtile = wave - kspl * rt;
   extern __shared__ float merge_lds[];  // (ksplit - 1) * rt slots, sized at launch (none without key splits)
-  int worker, r;
-  long long rstart;
-  ReqWork w;
-  const Plan pl = plan_and_locate(a, lane, worker, r, rstart, w);
-  long long pos = (long long)worker * pl.chunk;
-  const long long end = min(pos + pl.chunk, pl.total);
-  if (pos >= end || r >= a.num_seqs) return;
-  int seglen = seg_units(a, w);
-  int seg = (int)udiv_plan(pos - rstart, seglen), off = (int)(pos - rstart - (long long)seg * seglen);
-  bool whole = !cuttable(a, w);
   int solo = 0;  // pieces run by a single wavefront so far (uniform across the workgroup)
-  while (pos < end) {
-    const long long seg_start = rstart + (long long)seg * seglen;
-    const int take = (int)min((long long)(seglen - off), end - pos);
-    // the segment's first seg_cost units stand for its fixed cost, the rest for its tiles: pieces are
-    // the workers' shares of the tile units (a worker holding only fixed-cost units has no piece, and
-    // the pieces are numbered from the worker holding the first tile). Uncut (whole): the worker where
-    // the segment starts runs all of it, one piece.
-    const int fc = a.seg_cost;
-    const long long first = whole ? worker : udiv_plan(seg_start + fc, pl.chunk);
-    const long long last = whole ? worker : udiv_plan(seg_start + seglen - 1, pl.chunk);
-    const int kvh = seg / w.rgroups, rg = seg % w.rgroups;
-    const int row0 = (rg * a.rt + rtile) * 16;
-    const int c0 = whole ? 0 : max(off - fc, 0);
-    const int c1 = whole ? (off == 0 ? w.ntiles : 0) : max(off + take - fc, 0);
+  walk_pieces(a, lane, [&](int r, const ReqWork& w, int kvh, int rg, int c0, int c1, int part, int nparts) {
+    const int row0 = (rg * rt + rtile) * 16;
     // a piece long enough for every key split to stream COOP_TILES tiles is split across them and
     // merged; shorter pieces go whole to one key split in turn (no barrier, no merge)
-    if (c1 <= c0) {
-      // fixed-cost units only: nothing to stream here (uniform across the workgroup)
-    } else if (a.ksplit > 1 && c1 - c0 >= a.ksplit * COOP_TILES) {
-      attend_segment<D, PF>(a, r, w.tok, w.qlen, w.len, kvh, row0, c0, c1, kspl, a.ksplit, rtile, row0 < w.qlen * a.G,
-                            (int)(worker - first), (int)(last - first + 1), merge_lds, lane);
+    if (ksplit > 1 && c1 - c0 >= ksplit * COOP_TILES) {
+      attend_segment<D, PF>(r, w.tok, w.qlen, w.len, kvh, row0, c0, c1, kspl, ksplit, rtile, part, nparts, merge_lds, lane);
     } else {
-      if (solo % a.ksplit == kspl)
-        attend_segment<D, PF>(a, r, w.tok, w.qlen, w.len, kvh, row0, c0, c1, 0, 1, rtile, row0 < w.qlen * a.G,
-                              (int)(worker - first), (int)(last - first + 1), merge_lds, lane);
+      if (solo % ksplit == kspl)
+        attend_segment<D, PF>(r, w.tok, w.qlen, w.len, kvh, row0, c0, c1, 0, 1, rtile, part, nparts, merge_lds, lane);
       ++solo;
     }
-    pos += take;
-    off = 0;
-    if (++seg == a.hkv * w.rgroups && pos < end) {  // on to the next request with work
-      rstart += (long long)seglen * a.hkv * w.rgroups;
-      seg = 0;
-      do {
-        if (++r >= a.num_seqs) return;
-        w = req_work(a, r);
-      } while (w.ntiles == 0);
-      seglen = seg_units(a, w);
-      whole = !cuttable(a, w);
-    }
-  }
+  });
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1268,10 +1329,11 @@ __device__ __forceinline__ void v32_prio() {
   }
 }
 template <int D, int PF, int QG, int KS>
-__device__ __forceinline__ void attend_rows32(const AttnArgs& a, int seq, int tok, int qlen, int seqlen, int kvh, int row0,
-                                              int c_begin, int c_end, int wave, int kw, bool active, int part,
-                                              int nparts, uint8_t* ring, float* vsl, float* ksl, float* merge,
-                                              int lane) {
+__device__ __forceinline__ void attend_rows32(int seq, int tok, int qlen, int seqlen, int kvh, int row0, int c_begin,
+                                              int c_end, int wave, int kw, int part, int nparts, uint8_t* ring,
+                                              float* vsl, float* ksl, float* merge, int lane) {
+  const AttnArgs& a = fresh_args();
+  const bool active = row0 < qlen * a.G;
   constexpr int KST = D / 32;       // 32-channel QK steps = 32-channel PV tiles
   constexpr int CHR = D / 16;       // 16-byte chunks per K (or V) row
   constexpr int RPI = WAVE / CHR;   // rows per DMA instruction
@@ -1371,7 +1433,7 @@ __device__ __forceinline__ void attend_rows32(const AttnArgs& a, int seq, int to
   // scales, and the V scales the epilogue reads (staged in this wavefront's LDS slice) -- are issued
   // before the first tiles' page ids and DMAs: vmcnt counts in issue order, so waiting for them does not
   // wait for the DMAs, and the three round trips overlap instead of adding up ----
-  const int R = row0 + n, rtok = R / G, rh = R % G;
+  const int R = row0 + n, rtok = div_group(a, R), rh = R - rtok * G;
   static_assert(QG == 0 || QG == 32, "q scales per row or per 32 channels");
   i32x4 qop[KST];
   float rs;
@@ -1621,7 +1683,7 @@ __device__ __forceinline__ void attend_rows32(const AttnArgs& a, int seq, int to
   // compile-time slots, then the rest); wavefronts may split their steps differently between the loops
   // but each meets exactly nsteps barriers. ----
   if (nt > 0) {
-    const int lim_lo = L - qlen + 1 + row0 / G;          // every row of this wavefront sees keys < lim_lo
+    const int lim_lo = L - qlen + 1 + __builtin_amdgcn_readfirstlane(div_group(a, row0));          // every row of this wavefront sees keys < lim_lo
     const int full_end = lim_lo > 0 ? lim_lo / TILE : 0;
     const int j_full = work ? max(0, min(nt, full_end - c_begin)) : nt;
     const int i_full = j_full > kw ? (j_full - kw + KS - 1) / KS : 0;   // the split's unmasked tiles
@@ -1744,6 +1806,7 @@ __device__ __forceinline__ void attend_rows32(const AttnArgs& a, int seq, int to
 // wavefronts of key split 0.
 template <int D, int PF, int QG, int KS>
 __global__ __launch_bounds__(WAVE * 2 * KS) void verify_kernel(AttnArgs a) {
+  touch_args();
   const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int rw = wave & 1, kw = wave >> 1;
   extern __shared__ float v32_lds[];
@@ -1753,42 +1816,11 @@ __global__ __launch_bounds__(WAVE * 2 * KS) void verify_kernel(AttnArgs a) {
   float* vsl = reinterpret_cast<float*>(rings + v32_vscale_offset(D, PF, KS)) + rw * D;
   float* ksl = reinterpret_cast<float*>(rings + v32_vscale_offset(D, PF, KS)) + (2 + wave) * D;
   float* merge = reinterpret_cast<float*>(rings);
-  int worker, r;
-  long long rstart;
-  ReqWork w;
-  const Plan pl = plan_and_locate(a, lane, worker, r, rstart, w);
-  long long pos = (long long)worker * pl.chunk;
-  const long long end = min(pos + pl.chunk, pl.total);
-  if (pos >= end || r >= a.num_seqs) return;
-  int seglen = seg_units(a, w);
-  int seg = (int)udiv_plan(pos - rstart, seglen), off = (int)(pos - rstart - (long long)seg * seglen);
-  bool whole = !cuttable(a, w);
-  while (pos < end) {
-    const long long seg_start = rstart + (long long)seg * seglen;
-    const int take = (int)min((long long)(seglen - off), end - pos);
-    const int fc = a.seg_cost;
-    const long long first = whole ? worker : udiv_plan(seg_start + fc, pl.chunk);
-    const long long last = whole ? worker : udiv_plan(seg_start + seglen - 1, pl.chunk);
-    const int kvh = seg / w.rgroups, rg = seg % w.rgroups;
+  walk_pieces(a, lane, [&](int r, const ReqWork& w, int kvh, int rg, int c0, int c1, int part, int nparts) {
     const int row0 = rg * (16 * V32_GROUP_TILES) + 32 * rw;
-    const int c0 = whole ? 0 : max(off - fc, 0);
-    const int c1 = whole ? (off == 0 ? w.ntiles : 0) : max(off + take - fc, 0);
-    if (c1 > c0)
-      attend_rows32<D, PF, QG, KS>(a, r, w.tok, w.qlen, w.len, kvh, row0, c0, c1, rw, kw, row0 < w.qlen * a.G,
-                                   (int)(worker - first), (int)(last - first + 1), ring, vsl, ksl, merge, lane);
-    pos += take;
-    off = 0;
-    if (++seg == a.hkv * w.rgroups && pos < end) {  // on to the next request with work
-      rstart += (long long)seglen * a.hkv * w.rgroups;
-      seg = 0;
-      do {
-        if (++r >= a.num_seqs) return;
-        w = req_work(a, r);
-      } while (w.ntiles == 0);
-      seglen = seg_units(a, w);
-      whole = !cuttable(a, w);
-    }
-  }
+    attend_rows32<D, PF, QG, KS>(r, w.tok, w.qlen, w.len, kvh, row0, c0, c1, rw, kw, part, nparts, ring, vsl, ksl, merge,
+                                 lane);
+  });
 }
 
 // Merge the pieces of the cut segments (reference kvq/cuda/int8_kv.cu:465-503):
@@ -3624,6 +3656,8 @@ int decode_attention(const void* q, int64_t q_st, int64_t q_sh, const int8_t* k_
   a.seg_st = seg_st; a.seg_sh = seg_sh; a.bt_stride = bt_stride;
   a.sm_log2 = (float)(softmax_scale * 1.4426950408889634);
   a.num_blocks = (int)num_blocks; a.lbs = log2i(block_size); a.G = G;
+  // row indexes stay below G x (longest short query) + 64: exact by multiplication while that times G is below 2^32
+  a.g_inv = G > 1 && (G * std::min<int64_t>(qmax, INT32_MAX) + 64) < (1ll << 32) / G ? (unsigned)(((1ll << 32) + G - 1) / G) : 0u;
   a.qmax = (int)std::min<int64_t>(qmax, INT32_MAX);
   a.ks_pc = k_scale_cols > 1; a.vs_pc = v_scale_cols > 1;
   a.num_seqs = (int)num_seqs; a.hkv = (int)num_kv_heads;

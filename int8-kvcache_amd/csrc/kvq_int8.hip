@@ -50,7 +50,7 @@ constexpr int WAVE = 64;
 constexpr int TILE = 32;          // keys per attention tile = P quantization tile
 constexpr int MAX_SPLITS = 64;    // split_reduce_kernel keeps one split per lane
 constexpr int MAX_ROW_TILES = 4;  // row tiles (wavefronts) per attention workgroup
-constexpr int MIN_SPLIT_TILES = 4;  // shortest split: 4 tiles = 128 keys
+constexpr int MIN_SPLIT_TILES = 4;  // shortest piece of a cut segment: 4 tiles = 128 keys (below)
 constexpr int DEFAULT_WAVES_PER_CU = 8;
 constexpr int DEFAULT_KSPLIT = 2;     // key splits per row tile: skewed batches (c4) run 9% faster
                                       // than with 4 (2-wavefront workgroups, twice as many); c2 the same
@@ -540,6 +540,7 @@ struct AttnArgs {
   int num_blocks, lbs, ks_pc, vs_pc;
   unsigned g_inv;     // ceil(2^32 / G) where R / G = umulhi(R, g_inv) for every row index R of the call, else 0
   int ksplit;         // key splits per workgroup: wavefront (t, k) takes every ksplit-th key tile of row tile t
+  int coop;           // shortest piece split across the key splits, in tiles
   int waves;          // rt * ksplit wavefronts per workgroup
 };
 static_assert(offsetof(AttnArgs, q) == 64, "the plan's arguments fill the first 64 bytes");
@@ -874,10 +875,18 @@ __device__ __forceinline__ void transpose4x4(uint32_t a0, uint32_t a1, uint32_t 
 // denominator and accumulators in slot (k - 1) * rt + t, lane-major ([field][lane]: conflict-free).
 constexpr int MERGE_FIELDS = 36;  // 32 accumulators (D = 128), max, denominator, 2 spare
 constexpr int MERGE_SLOTS = MAX_ROW_TILES - 1;
-// Shortest piece split across a workgroup's key splits, in tiles per key split: shorter pieces go
-// whole to one key split in turn (no barrier, no merge). c4's decode rows: 2, 3, 4 all 117.8-118.0 us,
-// 6 119.0, 8 119.3, 16 121.9 us.
+// Shortest piece of a cut segment, and the shortest a workgroup splits across its key splits (others go whole to
+// one key split in turn: no barrier, no merge), in tiles: 4 each. In graphs, same box, against 8 and 8 (28 / 4 heads
+// unless said): 1 x 1,000 keys 12.6 -> 11.6 us, 4 x 500 13.7 -> 11.7, 8 x 2k 17.0 -> 15.9, 16 x 100 12.7 -> 11.8, 4 x 14k
+// 27.2 -> 26.0, c4's 96 ragged rows 99.2 -> 98.7; 2 and 6 tiles time between the two. Pieces of one pass (nothing
+// cut) are split from 4 tiles per key split on, and verify_kernel cuts no piece below 4 tiles per key split.
 constexpr int COOP_TILES = 4;
+constexpr int COOP_TILES_ONE_PASS = 16;
+// Up to this many (request, kv head) pairs a decode workgroup holds 4 key splits instead of 2: few pieces, so more
+// wavefronts on each (same box, 2 and 4: 1 x 32k 35.8 and 28.6 us, 4 x 14k 26.0 and 24.1, 16 x 3k of 14 / 2 heads d64
+// 14.6 and 13.8, 16 x 2k 18.5 and 18.1, 8 x 2k 15.9 and 15.8; 12 x 4k of 32 / 8 heads, 96 pairs, 23.5 and 23.9; 48 ragged
+// of 32 / 8, 384 pairs, 34.8 and 37.1).
+constexpr int WIDE_SPLIT_PAIRS = 64;
 constexpr float ATTN_SLACK = 8.f;  // log2 headroom of the attention's reference maximum
 
 // The end of a piece: lane group g writes channels (D/4) g .. + D/4 - 1 of its row (token qt, q head `head`) -- bf16
@@ -1243,8 +1252,8 @@ __device__ __forceinline__ void attend_segment(int seq, int tok, int qlen, int s
 // 16-row tiles (more than one only with KVQ_ROWS32=0: they stream the same K/V tiles at the same time, the
 // second and later reads hit L1/L2), each over ks interleaved sets of key tiles merged through LDS at the end of the piece.
 // Decode rows (one row tile) use 2 key splits, so a workgroup covers 2x the keys of one wavefront and
-// a long request's (kv head) is cut across workgroups half as often. Pieces too short for every key
-// split to stream COOP_TILES tiles are not split: the key splits take them in turn, each alone.
+// a long request's (kv head) is cut across workgroups half as often. Pieces shorter than a.coop tiles are
+// not split: the key splits take them in turn, each alone.
 template <int D, int PF>
 __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
   touch_args();
@@ -1256,9 +1265,8 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
   int solo = 0;  // pieces run by a single wavefront so far (uniform across the workgroup)
   walk_pieces(a, lane, [&](int r, const ReqWork& w, int kvh, int rg, int c0, int c1, int part, int nparts) {
     const int row0 = (rg * rt + rtile) * 16;
-    // a piece long enough for every key split to stream COOP_TILES tiles is split across them and
-    // merged; shorter pieces go whole to one key split in turn (no barrier, no merge)
-    if (ksplit > 1 && c1 - c0 >= ksplit * COOP_TILES) {
+    // a piece of at least a.coop tiles is split across the key splits and merged; shorter pieces go whole to one key split in turn (no barrier, no merge)
+    if (ksplit > 1 && c1 - c0 >= a.coop) {
       attend_segment<D, PF>(r, w.tok, w.qlen, w.len, kvh, row0, c0, c1, kspl, ksplit, rtile, part, nparts, merge_lds, lane);
     } else {
       if (solo % ksplit == kspl)
@@ -3630,7 +3638,7 @@ int decode_attention(const void* q, int64_t q_st, int64_t q_sh, const int8_t* k_
   // Without split buffers nothing is cut across workgroups: as many key splits as the workgroup
   // holds then run each segment
   const int ks_max = tune.ksplit ? std::max(1, std::min(MAX_ROW_TILES, atoi(tune.ksplit)))
-                            : (num_splits == 1 ? MAX_ROW_TILES : DEFAULT_KSPLIT);
+                            : num_splits == 1 || num_seqs * num_kv_heads <= WIDE_SPLIT_PAIRS ? MAX_ROW_TILES : DEFAULT_KSPLIT;
   const int ks = std::max(1, std::min(ks_max, MAX_ROW_TILES / rt));
   // more than one 16-row tile per (request, kv head): the 32-row wavefronts of verify_kernel, whose row
   // wavefronts share each K/V tile through LDS (KVQ_ROWS32=0: off). Two row tiles of attn_kernel each stream
@@ -3664,7 +3672,8 @@ int decode_attention(const void* q, int64_t q_st, int64_t q_sh, const int8_t* k_
   a.max_splits = (int)num_splits;
   a.cut_rows = num_splits > 1 ? (int)std::min<int64_t>(segm_rows, INT32_MAX) : 0;
   a.rt = rows32 ? V32_GROUP_TILES : rt; a.ksplit = rows32 ? v32ks : ks; a.waves = waves;
-  a.min_tiles = MIN_SPLIT_TILES * a.ksplit;
+  a.min_tiles = rows32 ? MIN_SPLIT_TILES * a.ksplit : MIN_SPLIT_TILES;
+  a.coop = num_splits == 1 ? COOP_TILES_ONE_PASS : COOP_TILES;
   a.xcd_order = tune.xcd_order ? atoi(tune.xcd_order) : 1;
   // KVQ_PLAN_FAST_MAX (tests): a lower bound on units sends the plan's scans down the 64-bit path
   a.plan_fast_max = tune.plan_fast_max ? (int)std::max(1ll, std::min(PLAN_FAST_MAX, atoll(tune.plan_fast_max)))

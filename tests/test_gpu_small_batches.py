@@ -35,3 +35,37 @@ def test_workgroup_order_of_small_batches(batch, q_len, monkeypatch):
                                         segm=nan_segm(d["q"].shape[0], 14, 16, 128), max_query_len=q_len))
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
     check_attention(oracle_attention(c, kq, vq), outs[0], "small_batch_order", batch=batch, q_len=q_len)
+
+
+@pytest.mark.parametrize("n", [1, 9, 32, 33])
+@pytest.mark.parametrize("heads", [(14, 2), (2, 2), (10, 2)])
+@pytest.mark.parametrize("segm", [False, True])
+def test_key_splits_at_their_edges(n, heads, segm):
+    """Pieces of 1 to 9 tiles around the shortest that is cut and the shortest that the key splits share (4 tiles),
+    with 4 key splits (up to 64 pairs: 32 requests of 2 kv heads) and 2 (33), cut or in one pass."""
+    hq, hkv = heads
+    lens = [(1, 32, 33, 96, 127, 128, 129, 160, 257, 288)[i % 10] for i in range(n)]
+    params = synth.channel_params(hkv, 128)
+    c = synth.paged_case(hq, hkv, [1] * n, lens, seed=50 + n, params=params)
+    c["static"] = synth.calibration_scales(hkv, 128, params)
+    c["scale"] = 128 ** -0.5
+    kq, vq = int8_cache(c)
+    d = dev(c)
+    out = ck.decode_attention(d["q"], dev(kq), dev(vq), nan_like(d["q"]), d["cu"], d["seq_lens"], d["block_table"],
+                              c["scale"], d["static"], segm=nan_segm(n, hq, 16, 128) if segm else None)
+    check_attention(oracle_attention(c, kq, vq), out, "key_split_edges", n=n, heads=list(heads), segm=segm)
+
+
+@pytest.mark.parametrize("heads,q_lens", [((1, 1), [1, 8]), ((71, 1), [1, 2]), ((3, 1), [8, 5]), ((127, 1), [8])])
+def test_row_to_token_division(heads, q_lens):
+    """(token, q head) rows of 1, 3, 71 and 127 q heads per kv head: the row's token comes from a multiplication."""
+    hq, hkv = heads
+    params = synth.channel_params(hkv, 128)
+    c = synth.paged_case(hq, hkv, q_lens, [300 + 7 * i for i in range(len(q_lens))], seed=60 + hq, params=params)
+    c["static"] = synth.calibration_scales(hkv, 128, params)
+    c["scale"] = 128 ** -0.5
+    kq, vq = int8_cache(c)
+    d = dev(c)
+    out = ck.decode_attention(d["q"], dev(kq), dev(vq), nan_like(d["q"]), d["cu"], d["seq_lens"], d["block_table"],
+                              c["scale"], d["static"], segm=nan_segm(sum(q_lens), hq, 16, 128), max_query_len=max(q_lens))
+    check_attention(oracle_attention(c, kq, vq), out, "row_division", heads=list(heads))

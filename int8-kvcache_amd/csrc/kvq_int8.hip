@@ -1979,16 +1979,22 @@ __device__ __forceinline__ u32x4 dq8x(uint32_t w0, uint32_t w1, const float (&s)
 // lanes' stores are consecutive: each store instruction writes whole rows of the output [P, bs, H, D]
 // (16 lanes per 256-byte K or V row at D = 128), never parts of lines.
 constexpr int DQ_BATCH = 16;
+// Few pages leave CUs idle and their workgroups a serial run of tokens, so a page's tokens are split over grid.z
+// down to DQ_MIN_TOKENS, up to about DQ_WG_PER_CU workgroups per CU (whole prefill calls in a graph, same box: 479
+// tokens of 498, 32 / 8 heads, blocks of 64 slots 30.4 -> 22.7 us, 157 of 157, 16 / 16 heads d64 19.8 -> 11.7, 1,024 of
+// 1,024 in blocks of 32 34.6 -> 33.3; 512 pages of 16 slots unchanged; slices of 16 tokens 23.8 and 12.7).
+constexpr int DQ_WG_PER_CU = 4, DQ_MIN_TOKENS = 4;
 template <int D>
 __global__ __launch_bounds__(256) void dequant_pages_kernel(
     const int8_t* __restrict__ kc, int64_t k_sb, int64_t k_sn, int64_t k_sh, const int8_t* __restrict__ vc,
     int64_t v_sb, int64_t v_sn, int64_t v_sh, int num_blocks, int bs, int H, int heads_per_block,
-    uint16_t* __restrict__ ko, uint16_t* __restrict__ vo, const int* __restrict__ bt, int64_t bt_stride,
+    int tokens_per_block, uint16_t* __restrict__ ko, uint16_t* __restrict__ vo, const int* __restrict__ bt, int64_t bt_stride,
     const int* __restrict__ src_req, const int* __restrict__ src_j, const float* __restrict__ ks, int ks_pc,
     const float* __restrict__ vs, int vs_pc) {
   constexpr int CPK = D / 8;                      // 8-channel chunks of one K (or V) row
   constexpr int CPH = 2 * CPK;                    // combinations per head: K and V chunks
   const int p = blockIdx.x;
+  const int z0 = blockIdx.z * tokens_per_block, z1 = min(bs, z0 + tokens_per_block);   // this workgroup's tokens
   const int h0 = blockIdx.y * heads_per_block;
   const int nh = min(heads_per_block, H - h0);
   const int C = nh * CPH;
@@ -2016,17 +2022,17 @@ __global__ __launch_bounds__(256) void dequant_pages_kernel(
   const int8_t* base = kv ? vc + (int64_t)src * v_sb + (int64_t)h * v_sh + d0 : kc + (int64_t)src * k_sb + (int64_t)h * k_sh + d0;
   const int64_t tstride = kv ? v_sn : k_sn;
   uint16_t* obase = (kv ? vo : ko) + ((int64_t)p * bs * H + h) * D + d0;
-  for (int tb = t0; tb < bs; tb += DQ_BATCH * tpc) {
+  for (int tb = z0 + t0; tb < z1; tb += DQ_BATCH * tpc) {
     u32x2 w[DQ_BATCH];
 #pragma unroll
     for (int i = 0; i < DQ_BATCH; ++i) {
       const int t = tb + i * tpc;
-      if (t < bs) w[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(base + t * tstride));
+      if (t < z1) w[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(base + t * tstride));
     }
 #pragma unroll
     for (int i = 0; i < DQ_BATCH; ++i) {
       const int t = tb + i * tpc;
-      if (t >= bs) break;
+      if (t >= z1) break;
       __builtin_nontemporal_store(dq8x(w[i].x, w[i].y, sc), reinterpret_cast<u32x4*>(obase + (int64_t)t * H * D));
     }
   }
@@ -3764,10 +3770,16 @@ int kvq_dequant_pages(const int8_t* k_cache, int64_t k_sb, int64_t k_sn, int64_t
   const int hpb = (int)std::min<int64_t>(num_heads, 256 / cph);
   const int combos = hpb * cph;
   const int threads = (256 / combos) * combos;
-  const dim3 grid((unsigned)num_pages, (unsigned)((num_heads + hpb - 1) / hpb));
+  // few pages: each page's tokens over several workgroups
+  const int64_t groups = (num_heads + hpb - 1) / hpb;
+  const int64_t want = std::max<int64_t>(1, (int64_t)device_cus() * DQ_WG_PER_CU / (num_pages * groups));
+  const int64_t tokens = std::max<int64_t>(std::min<int64_t>(DQ_MIN_TOKENS, block_size), (block_size + want - 1) / want);
+  const int64_t slices = (block_size + tokens - 1) / tokens;
+  if (slices > 65535) return fail("dequant_pages: block_size too large");
+  const dim3 grid((unsigned)num_pages, (unsigned)groups, (unsigned)slices);
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(threads), 0, st, k_cache, k_sb, k_sn, k_sh, v_cache, v_sb, v_sn, v_sh,
-                       (int)num_blocks, (int)block_size, (int)num_heads, hpb, (uint16_t*)k_out, (uint16_t*)v_out,
+                       (int)num_blocks, (int)block_size, (int)num_heads, hpb, (int)tokens, (uint16_t*)k_out, (uint16_t*)v_out,
                        block_table, bt_stride, src_req, src_j, k_scale, (int)(k_scale_cols > 1), v_scale,
                        (int)(v_scale_cols > 1));
   };

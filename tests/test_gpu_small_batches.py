@@ -5,7 +5,7 @@ from conftest import nan_like, nan_segm
 
 from kvq import cuda_kernels as ck
 from kvq import synth
-from test_gpu_kernels import check_attention, dev, int8_cache, oracle_attention
+from test_gpu_kernels import _check_dequant, _random_pages, check_attention, dev, int8_cache, oracle_attention
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +69,12 @@ def test_row_to_token_division(heads, q_lens):
     out = ck.decode_attention(d["q"], dev(kq), dev(vq), nan_like(d["q"]), d["cu"], d["seq_lens"], d["block_table"],
                               c["scale"], d["static"], segm=nan_segm(sum(q_lens), hq, 16, 128), max_query_len=max(q_lens))
     check_attention(oracle_attention(c, kq, vq), out, "row_division", heads=list(heads))
+
+
+@pytest.mark.parametrize("D,bs,pages,H", [(128, 64, 1, 8), (64, 128, 3, 5), (128, 256, 2, 3), (64, 32, 700, 16),
+                                          (128, 8, 1, 2), (128, 64, 300, 8)])
+@pytest.mark.parametrize("per_channel", [True, False])
+def test_dequant_token_slices_bit_exact(D, bs, pages, H, per_channel):
+    """Few pages: a page's tokens over several workgroups (slices of 4 tokens and up, a last one shorter)."""
+    kq, vq, bt, src_req, src_j, st = _random_pages(max(pages, 4), bs, H, D, pages, pages + bs, per_channel)
+    _check_dequant(kq, vq, bt, src_req, src_j, st)

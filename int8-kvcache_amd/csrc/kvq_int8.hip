@@ -1852,7 +1852,7 @@ __device__ __forceinline__ void merge_row(const AttnArgs& a, int tok, int t, int
   // the maxima and the first MERGE_SPEC pieces' partial outputs are fetched with the denominators (one
   // memory round trip for a row of up to MERGE_SPEC pieces), later pieces four at a time
   const bool held = lane < a.max_splits;
-  constexpr int CPL = D / WAVE, UNR = 4;
+  constexpr int CPL = D / WAVE;
   const float* po = a.segm_out + base * D + CPL * lane;
   const float enc = held ? a.segm_sum[base + lane] : -1.f;
   const float mraw = held ? a.segm_max[base + lane] : -INFINITY;
@@ -1889,7 +1889,8 @@ __device__ __forceinline__ void merge_row(const AttnArgs& a, int tok, int t, int
 #pragma unroll
     for (int e = 0; e < CPL; ++e) num[e] = in ? __builtin_fmaf(ws, v0[j][e], num[e]) : num[e];
   }
-  for (int s0 = MERGE_SPEC; s0 < S; s0 += UNR) {
+  auto pieces = [&](auto unr_t, int s0) {   // pieces s0 .. s0 + UNR - 1, requested together
+    constexpr int UNR = decltype(unr_t)::value;
     float v[UNR][CPL];
 #pragma unroll
     for (int j = 0; j < UNR; ++j) {  // pieces past the last re-read it (in bounds), unused
@@ -1904,7 +1905,13 @@ __device__ __forceinline__ void merge_row(const AttnArgs& a, int tok, int t, int
 #pragma unroll
       for (int e = 0; e < CPL; ++e) num[e] = in ? __builtin_fmaf(ws, v[j][e], num[e]) : num[e];
     }
-  }
+  };
+  // a row of many pieces (a small batch's) reads 8 at a time, one of few 4: in graphs, same box, 4 / 8 / 14 at a time
+  // 8 x 2k keys 15.8 / 15.5 / 15.3 us, 1 x 4,096 14.7 / 14.5 / 14.4, c4's decode rows 99.2 / 98.8 / 98.8, 64 x 8-token
+  // verification (few pieces a row) 56.1 / 55.8 / 56.6
+  int s0 = MERGE_SPEC;
+  for (; s0 + 4 < S; s0 += 8) pieces(std::integral_constant<int, 8>{}, s0);
+  for (; s0 < S; s0 += 4) pieces(std::integral_constant<int, 4>{}, s0);
   uint16_t* op = a.out + (int64_t)(tok + t) * a.o_st + (int64_t)h * a.o_sh + CPL * lane;
   if constexpr (CPL == 2) {
     *reinterpret_cast<uint32_t*>(op) = pack_bf16x2(num[0] * inv, num[1] * inv);

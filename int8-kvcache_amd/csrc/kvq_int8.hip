@@ -3792,7 +3792,6 @@ int kvq_dequant_pages(const int8_t* k_cache, int64_t k_sb, int64_t k_sn, int64_t
   const int64_t want = std::max<int64_t>(1, (int64_t)device_cus() * DQ_WG_PER_CU / (num_pages * groups));
   const int64_t tokens = std::max<int64_t>(std::min<int64_t>(DQ_MIN_TOKENS, block_size), (block_size + want - 1) / want);
   const int64_t slices = (block_size + tokens - 1) / tokens;
-  if (slices > 65535) return fail("dequant_pages: block_size too large");
   const dim3 grid((unsigned)num_pages, (unsigned)groups, (unsigned)slices);
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(threads), 0, st, k_cache, k_sb, k_sn, k_sh, v_cache, v_sb, v_sn, v_sh,

@@ -623,7 +623,7 @@ def long_attention(q, k_cache, v_cache, out, cu_seqlens_q, seq_lens, block_table
         debug_dump.dump_long_call(os.environ["KVQ_DEBUG_DUMP"], q, out, cu_seqlens_q, seq_lens, plan,
                                   (plan.src_req.shape[0], bs, h, d), *plan.tiles(q.shape[1] // h, q.device),
                                   max_query_len, e.prefill_rows, softmax_scale)
-    direct = os.environ.get("KVQ_PREFILL_DIRECT") or ("1" if work.direct else "0")
+    direct = os.environ.get("KVQ_PREFILL_DIRECT", "1" if work.direct else "0")
     _check(direct in ("0", "1", "fold"), f"KVQ_PREFILL_DIRECT must be 0, 1 or fold, got {direct!r}")
     ks, vs = static["k_scale"], static["v_scale"]
     src = plan.gpu(q.device) if direct == "0" else (None, None, None)

@@ -627,7 +627,7 @@ def main():
                    "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "achieved": round(alg / (launch_ms * 1e-3) / 1e9, 1), "peak": PEAK_GBS,
                      "unit": "GB/s", "frac": round(alg / (launch_ms * 1e-3) / 1e9 / PEAK_GBS, 4), "traffic": None,
-                     "kernel": "attn_kernel<128, 2, false> (one pass)",
+                     "kernel": "attn_kernel<128, 2> (one pass)",
                      "launch_us_timed_region": round(launch_ms * 1e3, 1),
                      "how": "algorithmic bytes / (HIP event interval around the timed region's launches / steps)",
                      "kernel_us_mean": round(kern_ms_mean * 1e3, 1), "kernel_us_median": round(kern_ms_med * 1e3, 1),

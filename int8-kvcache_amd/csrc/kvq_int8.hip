@@ -38,6 +38,7 @@
 #include <type_traits>
 
 #include "../../include/kvq_int8.h"
+#include "page_run.h"
 
 namespace {
 
@@ -2314,10 +2315,10 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
     if (lin) {
       // the upper half as below: past the last page (bs == 16) it re-reads the lower half's page
       const uint32_t k1 = ((min(kb0 + 16, klast) >> a.lbs) << a.lbs) + ((kb0 + 16) & bsm);
-      kb[0] = klin + (uint32_t)kb0 * a.krow;
-      vb[0] = vlin + (uint32_t)kb0 * a.vrow;
-      kb[1] = klin + k1 * a.krow;
-      vb[1] = vlin + k1 * a.vrow;
+      kb[0] = klin + run_offset(kb0, a.krow);
+      vb[0] = vlin + run_offset(kb0, a.vrow);
+      kb[1] = klin + run_offset(k1, a.krow);
+      vb[1] = vlin + run_offset(k1, a.vrow);
     } else {
       const int i0 = kb0 >> a.lbs, i1 = min(kb0 + 16, klast) >> a.lbs;
       int p0 = __builtin_amdgcn_readfirstlane(((const __attribute__((address_space(4))) int*)bt)[i0]);

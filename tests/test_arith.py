@@ -32,3 +32,10 @@ def test_division_free_codes_match_ieee_codes(tmp_path):
     bf16 absolute maxima / 127, a third putting a chosen x exactly on a tie)."""
     rc, out = _run_c(tmp_path, "quant_exact_check")
     assert rc == 0 and out.endswith("mismatched 0"), out
+
+
+def test_page_run_offsets_do_not_wrap(tmp_path):
+    """prefill_body's offset of a key within a run of consecutive pages (run_offset, csrc/page_run.h): the full
+    product, also more than 4 GiB from the run's first key (524,288 keys of 32 kv heads in the bf16 cache)."""
+    rc, out = _run_c(tmp_path, "page_run_check")
+    assert rc == 0 and out.endswith("mismatched 0"), out

@@ -96,3 +96,51 @@ def test_split_direct_prefill_bit_identical(d, layout, upper, monkeypatch):
     assert torch.equal(outs["0", 1.5].view(torch.int16), outs["1", 1.5].view(torch.int16))
     err = O.compare(outs["0", 0][long_rows], outs["0", 1.5][long_rows])
     assert err["max_abs"] <= 2e-2 and err["rel_l2"] < 5e-3, err            # bf16 P and output, sums in another order
+
+
+def _both_orders(src, hq, hkv, d, q_len, ids, parts, seed):
+    """One request over the pages `ids` (in this order) of a contiguous cache, cut into `parts` pieces, and the same
+    keys with the pages in another order, read through the block table: (out, out)."""
+    n = ids.shape[0]
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    shape = (n, 16, hkv, d)
+    if src == "int8":
+        k, v = (torch.randint(-127, 128, shape, generator=g, device=DEV, dtype=torch.int8) for _ in range(2))
+    else:
+        k, v = (torch.randn(shape, generator=g, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    st = [torch.rand(hkv, d, generator=g, device=DEV) * 0.02 + 1e-3 for _ in range(2)]
+    q = torch.randn(q_len, hq, d, generator=g, device=DEV, dtype=torch.bfloat16)
+    cu = torch.tensor([0, q_len], dtype=torch.int32, device=DEV)
+    sl = torch.tensor([16 * n - 3], dtype=torch.int32, device=DEV)
+    plan = ck.plan_long(np.array([0, q_len]), np.array([16 * n - 3]), 16)
+    tile_req, tile_row, split = _split(plan, hq // hkv, hkv, d, parts)
+    outs = []
+    for swap in (False, True):
+        if swap:    # a page moves to another place: pages i and n - 1 - i trade places, the table follows
+            k, v, ids = k.flip(0).contiguous(), v.flip(0).contiguous(), n - 1 - ids
+        out = nan_like(q)
+        args = (q, k, v, out, cu, sl, ids.to(device=DEV, dtype=torch.int32)[None].contiguous(), tile_req, tile_row, d ** -0.5)
+        if src == "int8":
+            ck.ext().int8_prefill_attention(*args, *st, split=split if parts > 1 else None)
+        else:
+            ck.ext().paged_prefill_attention(*args, split=split if parts > 1 else None)
+        outs.append(out)
+    return outs
+
+
+@pytest.mark.parametrize("src", ["bf16", "int8"])
+def test_piece_of_pages_with_low_ids(src):
+    """Pieces whose consecutive pages have ids below their place in the request: the run's key 0 would lie before
+    the cache. The last 63 pages are pages 0 .. 62, the 62 before them lie after those in a scattered order."""
+    ids = torch.cat([63 + (torch.arange(62) * 23) % 62, torch.arange(63)])
+    a, b = _both_orders(src, 28, 4, 128, 40, ids, 7, 1)
+    assert torch.isfinite(a.float()).all() and torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("parts", [1, 64])
+@pytest.mark.parametrize("src,hkv", [("bf16", 32), ("int8", 64)])
+def test_run_of_pages_longer_than_4_gib(src, hkv, parts):
+    """532,480 keys on consecutive pages, 4.06 GiB of K from the first key to the last: the offset of a key within
+    the run needs more than 32 bits."""
+    a, b = _both_orders(src, hkv, hkv, 128, 12, torch.arange((1 << 15) + 512), parts, 2)
+    assert torch.isfinite(a.float()).all() and torch.equal(a.view(torch.int16), b.view(torch.int16))

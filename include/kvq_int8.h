@@ -24,6 +24,9 @@
 
 #include <stdint.h>
 
+/* The version of these entry points' signatures (kvq_abi_version): changes with any of them. */
+#define KVQ_ABI_VERSION 12
+
 #ifdef __cplusplus
 extern "C" {
 #endif

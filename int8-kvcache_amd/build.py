@@ -6,6 +6,7 @@ this file's kvq/ package so that they travel with the source tree.
 """
 import importlib.util
 import os
+import re
 import subprocess
 import sys
 import sysconfig
@@ -31,12 +32,16 @@ CXX = os.environ.get("KVQ_CXX", "/opt/rocm/bin/amdclang++")
 
 def _calls_flags():
     torch_dir = os.path.dirname(importlib.util.find_spec("torch").origin)
+    with open(os.path.join(torch_dir, "version.py")) as f:   # torch.__version__ without importing torch
+        version = re.search(r"^__version__ = ['\"](.+)['\"]", f.read(), re.M).group(1)
     return ["-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-            f"-I{torch_dir}/include", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}",
+            f'-DKVQ_TORCH_VERSION="{version}"', f"-I{torch_dir}/include", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}",
             f"-L{torch_dir}/lib", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
 
 
 def build(verbose=False):
+    """Compile both. An output whose compilation failed is removed: a file of an earlier build beside a new one
+    would be called with signatures that are no longer the library's."""
     jobs = []
     for cmd, out in (([HIPCC, *FLAGS, SRC], OUT), ([CXX, CALLS_SRC, *_calls_flags()], CALLS_OUT)):
         cmd = [*cmd, "-o", out + ".tmp"]
@@ -48,6 +53,9 @@ def build(verbose=False):
         text = job.communicate()[0]
         if job.returncode != 0:
             failed.append(f"building {os.path.basename(out)} failed ({job.returncode}):\n{text[-4000:]}")
+            for path in (out, out + ".tmp"):
+                if os.path.exists(path):
+                    os.remove(path)
         else:
             os.replace(out + ".tmp", out)
     if failed:

@@ -3451,7 +3451,7 @@ int kvq_stream_scatter(const void* key, int64_t key_st, int64_t key_sh, const vo
   return launched("stream_scatter");
 }
 
-int kvq_abi_version(void) { return 12; }
+int kvq_abi_version(void) { return KVQ_ABI_VERSION; }
 
 int kvq_prefill_rows_per_tile(void) { return PR_ROWS; }
 

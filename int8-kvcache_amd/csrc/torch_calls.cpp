@@ -18,9 +18,20 @@
 
 #include "../../include/kvq_int8.h"
 
+#ifndef KVQ_TORCH_VERSION
+#error "KVQ_TORCH_VERSION: torch.__version__ of the headers in use (int8-kvcache_amd/build.py passes it)"
+#endif
+#define KVQ_TEXT_(x) #x
+#define KVQ_TEXT(x) KVQ_TEXT_(x)
+
 namespace {
 
 constexpr long DECLINED = -1;
+
+// What this file's calls were compiled against: the library's signatures, torch's tensor layout, the interpreter's
+// objects. kvq._native binds the module only where all three are the running ones.
+constexpr char BUILT_FOR[] = "abi " KVQ_TEXT(KVQ_ABI_VERSION) ", torch " KVQ_TORCH_VERSION ", python " KVQ_TEXT(
+    PY_MAJOR_VERSION) "." KVQ_TEXT(PY_MINOR_VERSION);
 
 // the library's entry points, by address (bind): whichever library file the package loaded
 decltype(&kvq_quant_cache) p_quant_cache;
@@ -300,5 +311,6 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_torch_calls", "kvq operators on t
 PyMODINIT_FUNC PyInit__torch_calls(void) {
   PyObject* m = PyModule_Create(&module);
   if (m) PyModule_AddIntConstant(m, "DECLINED", DECLINED);
+  if (m) PyModule_AddStringConstant(m, "BUILT_FOR", BUILT_FOR);
   return m;
 }

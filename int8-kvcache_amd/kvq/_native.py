@@ -5,6 +5,8 @@ stale, load() raises, so nothing silently runs another implementation.
 """
 import ctypes
 import os
+import sys
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libkvq_int8.so")
@@ -96,14 +98,28 @@ def error(name):
     return NativeError(f"{name}: {load().kvq_last_error().decode()}")
 
 
+def calls_built_for():
+    """What kvq._torch_calls has to be compiled for to be called from here (its BUILT_FOR)."""
+    import torch
+
+    return f"abi {ABI_VERSION}, torch {torch.__version__}, python {sys.version_info[0]}.{sys.version_info[1]}"
+
+
 def torch_calls():
     """kvq._torch_calls (csrc/torch_calls.cpp: the operators on torch tensors, host code only) bound to the loaded
-    library, or None where it is not built for this torch: the operators then run their Python checks and the
-    ctypes calls, with the same results."""
+    library, or None, with a warning, where it does not import or was compiled for other signatures of the library,
+    another torch or another Python (its calls and its view of a tensor are fixed when it is compiled): the
+    operators then run their Python checks and the ctypes calls, with the same results."""
     lib = load()
+    want, built = calls_built_for(), "an unknown build"
     try:
         from . import _torch_calls
-    except ImportError:
+        built = getattr(_torch_calls, "BUILT_FOR", built)
+    except ImportError as e:
+        built = str(e)
+    if built != want:
+        warnings.warn(f"kvq._torch_calls is not used ({built}; needs {want}): rebuild it with "
+                      "`python int8-kvcache_amd/build.py`", RuntimeWarning, stacklevel=2)
         return None
     _torch_calls.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES})
     return _torch_calls

@@ -575,6 +575,12 @@ def direct_pays(longest, d, elems):
     return TILE_DIRECT_US * _tile_unit(d) * longest < DEQUANT_US + elems / DEQUANT_ELEMS_PER_US
 
 
+def _direct_takes(cache):
+    """Whether the direct kernel's 32-bit page and slot offsets reach every byte of the cache's pages
+    (kvq_int8_prefill_attention refuses others; dequant_pages counts in 64 bits)."""
+    return cache.stride(0) < 1 << 32 and cache.shape[1] * cache.stride(1) < 1 << 31
+
+
 def plan_long(query_start_loc_cpu, seq_lens_cpu, block_size):
     """Page table of the temporary cache, or None when no request has more than SHORT_Q query
     tokens (reference kvq/cuda_kernels.py:80-103). Host lengths may be upper bounds: they only
@@ -613,7 +619,8 @@ def long_attention(q, k_cache, v_cache, out, cu_seqlens_q, seq_lens, block_table
     Rows of many keys may be cut into pieces and merged (LongPlan.work). KVQ_PREFILL_DIRECT (read at every
     call): 1 = one kernel reads the INT8 pages itself instead (int8_prefill_attention) -- no temporary cache,
     bit-identical output; fold = the same with the scales folded into q and the output (faster, not
-    bit-identical); 0 = the two kernels; unset = 1 or 0, whichever is faster (direct_pays)."""
+    bit-identical); 0 = the two kernels; unset = 1 or 0, whichever is faster (direct_pays), 0 where the pages
+    are too far apart for 1."""
     bs, h, d = k_cache.shape[1:]
     _check(bs == plan.block_size, f"block size {bs} != plan block size {plan.block_size}")
     e = ext()
@@ -623,7 +630,9 @@ def long_attention(q, k_cache, v_cache, out, cu_seqlens_q, seq_lens, block_table
         debug_dump.dump_long_call(os.environ["KVQ_DEBUG_DUMP"], q, out, cu_seqlens_q, seq_lens, plan,
                                   (plan.src_req.shape[0], bs, h, d), *plan.tiles(q.shape[1] // h, q.device),
                                   max_query_len, e.prefill_rows, softmax_scale)
-    direct = os.environ.get("KVQ_PREFILL_DIRECT", "1" if work.direct else "0")
+    direct = os.environ.get("KVQ_PREFILL_DIRECT")
+    if direct is None:
+        direct = "1" if work.direct and _direct_takes(k_cache) and _direct_takes(v_cache) else "0"
     _check(direct in ("0", "1", "fold"), f"KVQ_PREFILL_DIRECT must be 0, 1 or fold, got {direct!r}")
     ks, vs = static["k_scale"], static["v_scale"]
     src = plan.gpu(q.device) if direct == "0" else (None, None, None)

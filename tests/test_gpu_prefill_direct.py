@@ -6,6 +6,7 @@ runs the bf16 kernel's MFMA sequence, so the bar is bit-identity with the two-ke
 inputs (rows outside the work list stay NaN in both). The two-kernel path itself is checked against the
 oracle and fp32 attention in test_gpu_kernels.py and test_gpu_prefill.py.
 =fold: the scales folded into q and the output (tests at the end of this file)."""
+import numpy as np
 import pytest
 import torch
 from conftest import nan_like, record
@@ -306,3 +307,24 @@ def test_fold_score_jump(monkeypatch):
             worst = max(worst, (out[int(cu[r]) + t] - o).abs().max().item())
     record("prefill_fold_score_jump", max_abs=worst)
     assert torch.isfinite(out[:240]).all() and worst <= 2e-2, worst
+
+
+def test_pages_4_gib_apart_run_the_two_kernels(monkeypatch):
+    """Few rows, which the INT8 pages would serve directly, of a cache whose pages are more than 4 GiB apart."""
+    monkeypatch.delenv("KVQ_PREFILL_DIRECT", raising=False)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    stride = (1 << 32) + 4096
+    store = torch.empty(stride + 16 * 1024, dtype=torch.int8, device="cuda")
+    far = store.as_strided((2, 16, 4, 2 * 128), (stride, 1024, 256, 1))
+    far.copy_(torch.randint(-127, 128, far.shape, generator=g, device="cuda", dtype=torch.int8))
+    st = {k: torch.rand(4, 128, generator=g, device="cuda") * 0.02 + 1e-3 for k in ("k_scale", "v_scale")}
+    q = torch.randn(20, 28, 128, generator=g, device="cuda", dtype=torch.bfloat16)
+    cu, sl = (torch.tensor(x, dtype=torch.int32, device="cuda") for x in ([0, 20], [29]))
+    bt = torch.tensor([[1, 0]], dtype=torch.int32, device="cuda")
+    outs = []
+    for kv in (far, far.contiguous()):
+        out = torch.full_like(q, float("nan"))
+        plan = ck.plan_long(np.array([0, 20]), np.array([29]), 16)
+        ck.long_attention(q, kv[..., :128], kv[..., 128:], out, cu, sl, bt, 20, plan, 128 ** -0.5, st)
+        outs.append(out.view(torch.int16))
+    assert torch.equal(*outs)

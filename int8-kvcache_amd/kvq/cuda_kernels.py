@@ -406,6 +406,10 @@ def decode_attention(q, k_cache, v_cache, out, cu_seqlens_q, seq_lens, block_tab
     return out
 
 
+def _capturing(device):
+    return torch.device(device).type == "cuda" and torch.cuda.is_current_stream_capturing()
+
+
 def _to_device(arrays, device):
     """int32 device copies of the numpy arrays, in one transfer (each a view of one buffer, in this order)."""
     flat = torch.from_numpy(np.concatenate([x.reshape(-1) for x in arrays]).astype(np.int32, copy=False)).to(device)
@@ -462,11 +466,14 @@ class LongPlan:
     def work(self, group, hkv, d, device):
         """The prefill call's work list on the device (PrefillWork): `tiles`, the longest rows' keys cut into
         pieces where that pays (split_rows), and whether the call reads the INT8 pages itself. Built on the
-        host, copied once per plan and shape."""
+        host, copied once per plan and shape; a capture that finds it missing but `tiles` made takes those, whole
+        rows in two kernels, as nothing can be copied inside it."""
         if self._work is None:
             self._work = {}
         if (group, hkv, d) not in self._work:
             rows = ext().prefill_rows
+            if self._tiles and (group, rows) in self._tiles and _capturing(device):
+                return PrefillWork(*self._tiles[group, rows], None, None, None, 0, False)
             req, row, keys = self._row_tiles(group, rows)
             tiles = np.maximum((keys + PREFILL_TILE - 1) // PREFILL_TILE, 1)
             lists = split_rows(req, row, tiles, hkv, d, one_pass_fill(device), ext().prefill_max_parts)

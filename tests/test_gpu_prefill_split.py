@@ -144,3 +144,30 @@ def test_run_of_pages_longer_than_4_gib(src, hkv, parts):
     the run needs more than 32 bits."""
     a, b = _both_orders(src, hkv, hkv, 128, 12, torch.arange((1 << 15) + 512), parts, 2)
     assert torch.isfinite(a.float()).all() and torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+def test_capture_after_the_plans_own_copies(monkeypatch):
+    """A program that made the plan's device copies itself (gpu, tiles) and then captures its first call: the graph
+    holds the whole rows' two kernels; replays follow the inputs, and a later eager call agrees."""
+    monkeypatch.delenv("KVQ_PREFILL_DIRECT", raising=False)
+    g = torch.Generator().manual_seed(9)
+    nb, hq, hkv, d = 160, 28, 4, 128
+    kq, vq = (torch.randint(-127, 128, (nb, 16, hkv, d), generator=g, dtype=torch.int8).to(DEV) for _ in range(2))
+    st = {k: (torch.rand(hkv, d, generator=g) * 0.02 + 1e-3).to(DEV) for k in ("k_scale", "v_scale")}
+    q = torch.randn(20, hq, d, generator=g).to(torch.bfloat16).to(DEV)
+    cu, sl = (torch.tensor(x, dtype=torch.int32, device=DEV) for x in ([0, 20], [2500]))
+    bt = torch.randperm(nb, generator=g)[None].to(torch.int32).to(DEV)
+    plan = ck.plan_long(np.array([0, 20]), np.array([2500]), 16)
+    plan.gpu(DEV)
+    plan.tiles(hq // hkv, DEV)
+    out = nan_like(q)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ck.long_attention(q, kq, vq, out, cu, sl, bt, 20, plan, d ** -0.5, st)
+    for i in range(3):
+        q.normal_()
+        out.fill_(float("nan"))
+        graph.replay()
+        want = ck.long_attention(q, kq, vq, nan_like(q), cu, sl, bt, 20, plan, d ** -0.5, st)
+        err = O.compare(want.cpu(), out.cpu())
+        assert torch.isfinite(out.float()).all() and err["max_abs"] <= 2e-2 and err["rel_l2"] < 5e-3, (i, err)

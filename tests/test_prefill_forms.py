@@ -58,3 +58,20 @@ def test_pages_past_the_direct_kernels_offsets_take_the_two_kernels(wide, which,
 def test_the_last_page_stride_the_direct_kernel_takes(monkeypatch):
     last = (1 << 32) - 16
     assert _forms(monkeypatch, (last, 512, 128, 1), (last, (1 << 27) - 16, 128, 1)) == ["direct"]
+
+
+def test_lists_made_before_a_capture_serve_it(monkeypatch):
+    """A program that copied a plan's lists to the device itself (gpu, tiles) before it captures the call: nothing
+    may be copied inside the capture, so those lists serve it (whole rows, the two kernels)."""
+    e = Recorder()
+    monkeypatch.setattr(ck, "_EXT", e)
+    plan = ck.plan_long(np.array([0, 20]), np.array([5000]), 16)
+    plan.gpu("cpu")
+    tiles = plan.tiles(7, "cpu")
+    monkeypatch.setattr(ck, "_capturing", lambda device: True)
+    monkeypatch.setattr(ck, "_to_device", lambda *a: pytest.fail("a copy inside the capture"))
+    work = plan.work(7, 4, 128, torch.device("cpu"))
+    assert work.tile_req is tiles[0] and work.tile_row is tiles[1] and work.tile_piece is None and not work.direct
+    monkeypatch.undo()
+    monkeypatch.setattr(ck, "_EXT", e)
+    assert plan.work(7, 4, 128, torch.device("cpu")).tile_piece is not None     # outside it: the call's own list

@@ -38,6 +38,7 @@
 #include <type_traits>
 
 #include "../../include/kvq_int8.h"
+#include "attn_rules.h"
 #include "page_run.h"
 
 namespace {
@@ -1252,10 +1253,12 @@ __device__ __forceinline__ void attend_segment(int seq, int tok, int qlen, int s
   if (ks > 0 || !active || rtok >= qlen) return;
   finish_segment<D>(fresh_args(), kvh, tok + rtok, kvh * G + rh, g, m, l, acc, part, nparts);
 }
+
 // Stream-K attention: workgroup w walks units [w * chunk, (w + 1) * chunk) of the batch (the plan of
 // plan_and_locate), segment by segment. Its rt * ks wavefronts split each piece: rt consecutive
-// 16-row tiles (more than one only with KVQ_ROWS32=0: they stream the same K/V tiles at the same time, the
-// second and later reads hit L1/L2), each over ks interleaved sets of key tiles merged through LDS at the end of the piece.
+// 16-row tiles (two for 17 to 32 rows per kv head where verify_rows leaves them here, up to four with KVQ_ROWS32=0: they
+// stream the same K/V tiles at the same time, the second and later reads hit L1/L2), each over ks interleaved sets of
+// key tiles merged through LDS at the end of the piece.
 // Decode rows (one row tile) use 2 key splits, so a workgroup covers 2x the keys of one wavefront and
 // a long request's (kv head) is cut across workgroups half as often. Pieces shorter than a.coop tiles are
 // not split: the key splits take them in turn, each alone.
@@ -1282,8 +1285,8 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// Verification-shape attention: more than 16 (token, q head) rows per (request, kv head), e.g. 8
-// speculative tokens x 7 q heads = 56 rows. A workgroup of 2 x KS wavefronts takes a piece of one
+// Verification-shape attention: more than 32 (token, q head) rows per (request, kv head), e.g. 8
+// speculative tokens x 7 q heads = 56 rows, or more than 16 of many cut pairs (verify_rows). A workgroup of 2 x KS wavefronts takes a piece of one
 // (request, kv head, group of 64 rows): row wavefront rw owns rows row0 = 32 rw .. 32 rw + 31 of the
 // group, key split kw streams the piece's tiles kw, kw + KS, ...; the two row wavefronts of a key split
 // share each 32-key K/V tile through the split's LDS ring (wavefront rw DMAs keys 16 rw .. 16 rw + 15 of
@@ -3672,15 +3675,11 @@ int decode_attention(const void* q, int64_t q_st, int64_t q_sh, const int8_t* k_
   const int ks_max = tune.ksplit ? std::max(1, std::min(MAX_ROW_TILES, atoi(tune.ksplit)))
                             : num_splits == 1 || num_seqs * num_kv_heads <= WIDE_SPLIT_PAIRS ? MAX_ROW_TILES : DEFAULT_KSPLIT;
   const int ks = std::max(1, std::min(ks_max, MAX_ROW_TILES / rt));
-  // more than one 16-row tile per (request, kv head): the 32-row wavefronts of verify_kernel, whose row
-  // wavefronts share each K/V tile through LDS (KVQ_ROWS32=0: off). Two row tiles of attn_kernel each stream
-  // and transpose every tile themselves; graph, same box, 28 / 4 heads: 24 requests x 4 tokens (28 rows)
-  // 36.7 -> 25.3 us, 64 x 4 66.9 -> 54.2, 24 x 3 (21 rows) 30.4 -> 23.7, 16 x 5 of 32 / 8 heads (20 rows) 41.0 ->
-  // 28.9; 2 requests x 4 17.7 and 17.9. One row tile (decode) stays with attn_kernel: 96 ragged requests 101
-  // against 114 us there, 1 x 4,096 keys 14.9 against 16.8.
-  // (per-32-channel q scales run there for every row count)
-  const bool rows32 = q_group == 32 ||
-                      ((int64_t)G * maxq > 16 && !(tune.rows32 && atoi(tune.rows32) == 0));
+  // the 32-row wavefronts of verify_kernel (KVQ_ROWS32=0: off; per-32-channel q scales run there for every row
+  // count) or attn_kernel's 16-row tiles
+  const bool cuttable_any = num_splits > 1 && segm_rows > 0;
+  const bool rows32 = q_group == 32 || (verify_rows((int64_t)G * maxq, num_seqs * num_kv_heads, cuttable_any) &&
+                                        !(tune.rows32 && atoi(tune.rows32) == 0));
   const int v32ks = rows32 ? v32_key_splits(tune) : 1;
   const int waves = rows32 ? 2 * v32ks : rt * ks;
   if (num_seqs > INT32_MAX - 1 || num_kv_heads > 65535 || (num_q_heads + RED_WAVES - 1) / RED_WAVES > 65535 ||
@@ -3743,7 +3742,6 @@ int decode_attention(const void* q, int64_t q_st, int64_t q_sh, const int8_t* k_
   // CU an equal run of segments to stream in turn (uniform batches of 1, 2, 2.5 and 3 segments per CU
   // 36%, 1%, 19% and 15% faster, 4 per CU alike, 1.5 per CU 3% slower; c4's decode rows in one pass
   // 405 -> 252 us, c3 in one pass 162 -> 154 us).
-  const bool cuttable_any = num_splits > 1 && a.cut_rows > 0;
   const int64_t tw = target_waves > 0 ? target_waves
                    : cuttable_any     ? (int64_t)device_cus() * resident_waves((const void*)kern, WAVE * waves, lds)
                                       : (int64_t)device_cus() * waves;

@@ -39,3 +39,10 @@ def test_page_run_offsets_do_not_wrap(tmp_path):
     product, also more than 4 GiB from the run's first key (524,288 keys of 32 kv heads in the bf16 cache)."""
     rc, out = _run_c(tmp_path, "page_run_check")
     assert rc == 0 and out.endswith("mismatched 0"), out
+
+
+def test_short_query_kernel_rule(tmp_path):
+    """verify_rows (csrc/attn_rules.h): above 32 rows per kv head always verify_kernel; 17 to 32 rows only where
+    more than 16 (request, kv head) pairs may be cut into pieces; one row tile never."""
+    rc, out = _run_c(tmp_path, "attn_rules_check")
+    assert rc == 0 and out.endswith("mismatched 0"), out

@@ -20,6 +20,7 @@ KVQ_DEBUG=1 input check, so fixed-shape calls can be captured in a HIP graph.
 """
 import os
 from dataclasses import dataclass
+from typing import NamedTuple
 
 import numpy as np
 import torch
@@ -476,7 +477,13 @@ class LongPlan:
                 return PrefillWork(*self._tiles[group, rows], None, None, None, 0, False)
             req, row, keys = self._row_tiles(group, rows)
             tiles = np.maximum((keys + PREFILL_TILE - 1) // PREFILL_TILE, 1)
-            lists = split_rows(req, row, tiles, hkv, d, one_pass_fill(device), ext().prefill_max_parts)
+            held = self.long_qlen * group                                # a request's last entry may be part full
+            count = (held + rows - 1) // rows
+            valid = np.ones(req.shape[0])
+            valid[np.cumsum(count) - 1] = (held - (count - 1) * rows) / rows
+            elems = self.src_req.shape[0] * self.block_size * hkv * d
+            lists = split_rows(req, row, tiles, hkv, d, one_pass_fill(device), ext().prefill_max_parts,
+                               valid, elems)
             if lists is None:
                 order = np.argsort(-keys, kind="stable")
                 lists, longest, slots = (req[order], row[order]), int(tiles.max(initial=0)), 0
@@ -484,8 +491,7 @@ class LongPlan:
                 longest, slots = lists[5:]
                 lists = (lists[4], *lists[:4])   # the 16-byte merge entries first
             views = _to_device(lists, device)
-            pages = self.src_req.shape[0] * self.block_size * hkv * d
-            direct = direct_pays(longest, d, pages)
+            direct = direct_pays(longest, d, elems)
             self._work[(group, hkv, d)] = (PrefillWork(*views, None, None, None, 0, direct) if len(views) == 2 else
                                            PrefillWork(views[1], views[2], views[3], views[4], views[0], slots, direct))
         return self._work[(group, hkv, d)]
@@ -514,32 +520,58 @@ class PrefillWork:
 
 
 PREFILL_TILE = 32          # keys per tile of the prefill kernel
-PREFILL_MIN_PIECE = 4      # shortest piece, in tiles: a shorter one costs its start and merge more than it saves
+PREFILL_MIN_PIECE = 4      # a piece's length to aim at, in tiles: from there on a shorter one costs more than it saves
 PREFILL_PER_CU = 2         # pieces per CU a split work list may hold
 PREFILL_WHOLE = 1.5        # workgroups of whole rows per CU from which nothing is cut
-# us, measured at head_dim 128 (a tile costs 0.7 of it at 64, a piece half): a tile of a workgroup alone on its CU, the same with two
-# workgroups per CU, the same when the INT8 pages are converted in the kernel (beyond the first), the merge
-# launch, and a piece's partials (66 KB per kv head, written and read)
-TILE_US, TILE2_US, TILE_DIRECT_US, MERGE_US, PIECE_US = 0.6, 0.85, 0.38, 4.0, 0.02
-DEQUANT_US, DEQUANT_ELEMS_PER_US = 4.0, 0.85e6   # dequant_pages: its launch, K + V elements (6 bytes) per us
 
 
-def _tile_unit(d):
-    return 1.0 if d == 128 else 0.7
+class _PrefillCost(NamedTuple):
+    """us of a prefill call's parts at one head_dim: a least-squares fit of 1,060 drawn steps, each timed in a graph
+    in all four forms (rows whole or cut, pages dequantized first or read directly), 5% off on average."""
+    tile: float     # a key tile of a workgroup alone on its CU (a workgroup walks its tiles one after another)
+    shared: float   # more per tile with two workgroups per CU
+    direct: float   # more per tile where the kernel converts the INT8 pages
+    merge: float    # the merge launch (0.5 more than fitted: a cut that only just pays is not worth its buffers)
+    partial: float  # 128 rows' partials of one piece and kv head, written and read
+    dequant: float  # dequant_pages' launch, and its time per million K elements (with their V)
+    pages: float
 
 
-def split_rows(req, row, tiles, hkv, d, fill, max_parts):
+_COST = {128: _PrefillCost(0.64, 0.11, 0.37, 5.0, 0.038, 3.0, 1.4),
+         64: _PrefillCost(0.48, 0.07, 0.23, 3.7, 0.031, 3.0, 1.6)}
+
+
+def _cost(d):
+    return _COST.get(d, _COST[128])   # (the kernels refuse other head sizes)
+
+
+def _prefill_us(longest, workgroups, partials, d, fill, elems):
+    """Expected us of a call whose longest workgroup has `longest` tiles, beyond what every form costs: the cheaper of
+    the two sources, with `partials` x 128 rows of partials (None: rows whole, no merge)."""
+    c = _cost(d)
+    us = longest * (c.tile + (c.shared if workgroups > fill else 0))
+    us += 0 if partials is None else c.merge + c.partial * partials
+    return us + min(c.direct * longest, c.dequant + c.pages * elems / 1e6)
+
+
+def split_rows(req, row, tiles, hkv, d, fill, max_parts, valid=None, elems=0):
     """Cut the long rows of a prefill work list (request, first row, key tiles; one workgroup per entry and kv
     head) into pieces of key tiles: (req, row, piece | pieces << 16, slot, merge [cut rows, 4], longest piece,
-    slots), heaviest pieces first, or None where nothing is cut.
+    slots), heaviest pieces first, or None where nothing is cut. valid: each entry's rows in units of a full entry
+    (default: all full); elems: K elements a dequantization would convert.
 
     A workgroup walks its tiles one after another, so few rows over many keys leave most CUs idle. The pieces
     are the shortest that keep the list within PREFILL_PER_CU workgroups per CU (all resident, the CUs evenly
     loaded); a third per CU adds partials and merging without time (graph, 28 / 4 heads, 512 tokens of 8,192
-    keys: whole 169 us, 1 / 2 / 3 pieces per CU 106 / 90 / 103 us; 16 tokens of 16,384: 322 -> 39 us). Cut only
-    where the tiles saved are worth the partials and the merge: 1,024 tokens of 1,024 whole 34 us, cut 38; 256 of
-    256 16 and 19; 700 of 3,000 71 and 56; 128 of 1,000 31 and 28. From PREFILL_WHOLE workgroups per CU on the
-    rows balance among themselves: 448 workgroups (2,048 tokens from the start) 62 us whole, 64 cut."""
+    keys: whole 169 us, 1 / 2 / 3 pieces per CU 106 / 90 / 103 us; 16 tokens of 16,384: 322 -> 39 us). Each entry is
+    cut into equal shares of its tiles, so a piece may be shorter than that length (5 tiles aimed at 4: 3 and 2).
+    Cut only where the tiles saved are worth the partials and the merge (_prefill_us; us of the rows whole and cut,
+    each from the better source): 28 / 4 heads 1,024 tokens of 1,024 34 and 38, 700 of 3,000 71 and 56; 12 / 2 heads 817
+    of 831 26.9 and 30.7, 21 of 13,943 272 and 29; 14 / 2 heads d64 774 of 774, 374 of 396 and 25 20.7 and 23.8, 580 of
+    1,080 25.1 and 23.2. Over 1,860 drawn steps, 800 of them not among the fitted, the form taken is within 5% of the
+    fastest in 97 of 100 and takes more than 3% longer than whole rows in two kernels in 8 (at most 10%, 3 us). From PREFILL_WHOLE
+    workgroups per CU on the rows balance among themselves: 448 workgroups (2,048 tokens from the start) 62 us whole,
+    64 cut."""
     if req.shape[0] * hkv >= PREFILL_WHOLE * fill or req.shape[0] == 0:
         return None
     most, total, budget = int(tiles.max()), int(tiles.sum()), PREFILL_PER_CU * fill // hkv
@@ -555,11 +587,10 @@ def split_rows(req, row, tiles, hkv, d, fill, max_parts):
             lo = mid + 1
     parts = np.minimum((tiles + lo - 1) // lo, max_parts)
     cut = parts > 1
-    pieces = int(parts.sum()) * hkv
     longest = int(((tiles + parts - 1) // parts).max())
-    whole_us = TILE_US * _tile_unit(d) * most
-    cut_us = (TILE2_US if pieces > fill else TILE_US) * _tile_unit(d) * longest + MERGE_US + PIECE_US * d / 128 * pieces
-    if longest == most or cut_us >= whole_us:
+    partials = hkv * float((parts * cut * (1 if valid is None else valid)).sum())
+    if longest == most or (_prefill_us(longest, int(parts.sum()) * hkv, partials, d, fill, elems)
+                           >= _prefill_us(most, req.shape[0] * hkv, None, d, fill, elems)):
         return None
     at = np.repeat(np.arange(parts.shape[0]), parts)
     part = np.arange(at.shape[0]) - np.repeat(np.cumsum(parts) - parts, parts)
@@ -579,7 +610,8 @@ def direct_pays(longest, d, elems):
     over the pages and temporary cache. Graph, 28 / 4 heads, two kernels and direct: 64 tokens of 8,192 keys 37.4
     and 36.0 us, 16 of 16,384 39.2 and 30.8, 256 of 256 16.2 and 15.4; 512 of 8,192 90 and 108, 1,024 of 1,024
     34 and 40; 300 of 12,000 (16 / 16 heads, d64) 57 and 51."""
-    return TILE_DIRECT_US * _tile_unit(d) * longest < DEQUANT_US + elems / DEQUANT_ELEMS_PER_US
+    c = _cost(d)
+    return c.direct * longest < c.dequant + c.pages * elems / 1e6
 
 
 def _direct_takes(cache):

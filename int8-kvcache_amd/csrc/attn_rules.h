@@ -18,3 +18,11 @@
 static inline int verify_rows(int64_t rows, int64_t pairs, int cut) {
   return rows > 32 || (rows > 16 && cut && pairs > 16);
 }
+
+// Shortest piece attn_kernel splits across a workgroup's key splits, in tiles (shorter ones go whole to one key split
+// in turn: no barrier, no merge). Pieces of cut segments: 4 (graph, us, from 8 tiles on and from 4 on, 28 / 4 heads unless
+// said, the shortest worker share lowered with it: 1 x 1,000 keys 12.6 and 11.6, 4 x 500 13.7 and 11.7, 8 x 2k 17.0 and
+// 15.9, 16 x 100 12.7 and 11.8, 4 x 14k 27.2 and 26.0, c4's 96 ragged rows 99.2 and 98.7; 2 and 6 tiles time between the
+// two). Segments run whole: 4 per key split, the key splits having other segments to take in the meantime (16 tiles
+// at 2 key splits: 2 x 4 tokens of 14 / 2 heads d64 at up to 1,128 keys 11.5 -> 13.4, 69 x 4 at up to 463 13.0 -> 14.5).
+static inline int coop_tiles(int cut, int ksplit) { return cut ? 4 : 4 * ksplit; }

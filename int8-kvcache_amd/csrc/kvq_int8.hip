@@ -52,7 +52,8 @@ constexpr int WAVE = 64;
 constexpr int TILE = 32;          // keys per attention tile = P quantization tile
 constexpr int MAX_SPLITS = 64;    // split_reduce_kernel keeps one split per lane
 constexpr int MAX_ROW_TILES = 4;  // row tiles (wavefronts) per attention workgroup
-constexpr int MIN_SPLIT_TILES = 4;  // shortest piece of a cut segment: 4 tiles = 128 keys (below)
+constexpr int MIN_SPLIT_TILES = 4;  // shortest worker share of a batch that may be cut, in tiles (per key split in
+                                    // verify_kernel); a segment's last share may hold fewer of its tiles
 constexpr int DEFAULT_WAVES_PER_CU = 8;
 constexpr int DEFAULT_KSPLIT = 2;     // key splits per row tile: skewed batches (c4) run 9% faster
                                       // than with 4 (2-wavefront workgroups, twice as many); c2 the same
@@ -523,7 +524,7 @@ struct AttnArgs {
   int cut_rows;       // the split buffers' rows: tokens [0, cut_rows); a request with a token beyond is never cut
   int rt;             // row tiles per workgroup: consecutive 16-row tiles of one (request, kv head)
   int workers;        // workgroups of the attention grid
-  int min_tiles;      // shortest piece of a cut segment, in 32-key tiles
+  int min_tiles;      // shortest worker share where segments may be cut, in 32-key tiles (fixed cost included)
   int seg_cost;       // work units a segment costs beyond its tiles (its fixed start and finish)
   int xcd_order;      // map workgroups to workers XCD by XCD
   int plan_fast_max;  // the plan's scans run in 32 bits on DPP while every request's units are below this
@@ -877,13 +878,6 @@ __device__ __forceinline__ void transpose4x4(uint32_t a0, uint32_t a1, uint32_t 
 // denominator and accumulators in slot (k - 1) * rt + t, lane-major ([field][lane]: conflict-free).
 constexpr int MERGE_FIELDS = 36;  // 32 accumulators (D = 128), max, denominator, 2 spare
 constexpr int MERGE_SLOTS = MAX_ROW_TILES - 1;
-// Shortest piece of a cut segment, and the shortest a workgroup splits across its key splits (others go whole to
-// one key split in turn: no barrier, no merge), in tiles: 4 each. In graphs, same box, against 8 and 8 (28 / 4 heads
-// unless said): 1 x 1,000 keys 12.6 -> 11.6 us, 4 x 500 13.7 -> 11.7, 8 x 2k 17.0 -> 15.9, 16 x 100 12.7 -> 11.8, 4 x 14k
-// 27.2 -> 26.0, c4's 96 ragged rows 99.2 -> 98.7; 2 and 6 tiles time between the two. Pieces of one pass (nothing
-// cut) are split from 4 tiles per key split on, and verify_kernel cuts no piece below 4 tiles per key split.
-constexpr int COOP_TILES = 4;
-constexpr int COOP_TILES_ONE_PASS = 16;
 // Up to this many (request, kv head) pairs a decode workgroup holds 4 key splits instead of 2: few pieces, so more
 // wavefronts on each (same box, 2 and 4: 1 x 32k 35.8 and 28.6 us, 4 x 14k 26.0 and 24.1, 16 x 3k of 14 / 2 heads d64
 // 14.6 and 13.8, 16 x 2k 18.5 and 18.1, 8 x 2k 15.9 and 15.8; 12 x 4k of 32 / 8 heads, 96 pairs, 23.5 and 23.9; 48 ragged
@@ -3704,7 +3698,7 @@ int decode_attention(const void* q, int64_t q_st, int64_t q_sh, const int8_t* k_
   a.cut_rows = num_splits > 1 ? (int)std::min<int64_t>(segm_rows, INT32_MAX) : 0;
   a.rt = rows32 ? V32_GROUP_TILES : rt; a.ksplit = rows32 ? v32ks : ks; a.waves = waves;
   a.min_tiles = rows32 ? MIN_SPLIT_TILES * a.ksplit : MIN_SPLIT_TILES;
-  a.coop = num_splits == 1 ? COOP_TILES_ONE_PASS : COOP_TILES;
+  a.coop = coop_tiles(num_splits > 1, ks);
   a.xcd_order = tune.xcd_order ? atoi(tune.xcd_order) : 1;
   // KVQ_PLAN_FAST_MAX (tests): a lower bound on units sends the plan's scans down the 64-bit path
   a.plan_fast_max = tune.plan_fast_max ? (int)std::max(1ll, std::min(PLAN_FAST_MAX, atoll(tune.plan_fast_max)))

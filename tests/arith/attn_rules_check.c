@@ -1,4 +1,5 @@
-/* verify_rows over the sizes a call can have: one line per mismatch with the rule as the kernels were measured. */
+/* verify_rows and coop_tiles over the sizes a call can have: one line per mismatch with the rules as the kernels were
+   measured. */
 #include <stdio.h>
 
 #include "../../int8-kvcache_amd/csrc/attn_rules.h"
@@ -12,6 +13,11 @@ int main(void) {
         if (verify_rows(rows, pairs, cut) != want && ++bad < 5)
           printf("rows %ld pairs %ld cut %d: %d\n", (long)rows, (long)pairs, cut, !want);
       }
+  for (int ksplit = 1; ksplit <= 4; ++ksplit)
+    for (int cut = 0; cut < 2; ++cut, ++n) {
+      int want = cut ? 4 : 4 * ksplit;
+      if (coop_tiles(cut, ksplit) != want && ++bad < 5) printf("ksplit %d cut %d: %d\n", ksplit, cut, coop_tiles(cut, ksplit));
+    }
   printf("checked %ld mismatched %ld\n", n, bad);
   return bad != 0;
 }

@@ -43,6 +43,7 @@ def test_page_run_offsets_do_not_wrap(tmp_path):
 
 def test_short_query_kernel_rule(tmp_path):
     """verify_rows (csrc/attn_rules.h): above 32 rows per kv head always verify_kernel; 17 to 32 rows only where
-    more than 16 (request, kv head) pairs may be cut into pieces; one row tile never."""
+    more than 16 (request, kv head) pairs may be cut into pieces; one row tile never. coop_tiles: pieces are split
+    across the key splits from 4 tiles on, whole segments from 4 tiles per key split."""
     rc, out = _run_c(tmp_path, "attn_rules_check")
     assert rc == 0 and out.endswith("mismatched 0"), out

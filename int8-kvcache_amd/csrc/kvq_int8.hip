@@ -3344,7 +3344,7 @@ int kvq_paged_prefill_attention_ex(const void* q, int64_t q_st, int64_t q_sh, co
                                    const int32_t* tile_row, int64_t num_tiles, int64_t rows_per_tile,
                                    double softmax_scale, const int32_t* tile_piece, const int32_t* tile_slot,
                                    const int32_t* merge, int64_t num_merge, float* part_out, float* part_ml, void* stream) {
-  return prefill_launch("paged_prefill_attention_ex", 2, q, q_st, q_sh, k_cache, k_sb, k_sn, k_sh, v_cache, v_sb, v_sn,
+  return prefill_launch(tile_piece ? "paged_prefill_attention_ex" : "paged_prefill_attention", 2, q, q_st, q_sh, k_cache, k_sb, k_sn, k_sh, v_cache, v_sb, v_sn,
                         v_sh, num_blocks, block_size, num_kv_heads, head_dim, out, o_st, o_sh, cu_seqlens_q,
                         seq_lens, block_table, bt_stride, num_q_heads, tile_req, tile_row, num_tiles, rows_per_tile,
                         softmax_scale, nullptr, 1, nullptr, 1, 0,
@@ -3379,7 +3379,7 @@ int kvq_int8_prefill_attention_ex(const void* q, int64_t q_st, int64_t q_sh, con
                                   const int32_t* tile_piece, const int32_t* tile_slot, const int32_t* merge,
                                   int64_t num_merge, float* part_out, float* part_ml, void* stream) {
   if (fold_scales != 0 && fold_scales != 1) return fail("int8_prefill_attention_ex: fold_scales must be 0 or 1");
-  return prefill_launch("int8_prefill_attention_ex", 1, q, q_st, q_sh, k_cache, k_sb, k_sn, k_sh, v_cache, v_sb, v_sn,
+  return prefill_launch(tile_piece ? "int8_prefill_attention_ex" : "int8_prefill_attention", 1, q, q_st, q_sh, k_cache, k_sb, k_sn, k_sh, v_cache, v_sb, v_sn,
                         v_sh, num_blocks, block_size, num_kv_heads, head_dim, out, o_st, o_sh, cu_seqlens_q,
                         seq_lens, block_table, bt_stride, num_q_heads, tile_req, tile_row, num_tiles, rows_per_tile,
                         softmax_scale, k_scale, k_scale_cols, v_scale, v_scale_cols, fold_scales,

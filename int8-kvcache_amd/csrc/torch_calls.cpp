@@ -85,10 +85,14 @@ bool index_vector(const at::Tensor& t) { return t.dim() == 1 && t.scalar_type() 
 
 void* stream_of(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
+// The entry point this thread's last call went to (its own record: the interpreter lock is not held meanwhile).
+thread_local const char* entry = "";
+
 // The C call with the interpreter lock released (as ctypes does): a full launch queue blocks this thread alone.
 template <typename F>
-long launch(F&& f) {
+long launch(const char* name, F&& f) {
   long rc;
+  entry = name;
   Py_BEGIN_ALLOW_THREADS
   rc = f();
   Py_END_ALLOW_THREADS
@@ -129,7 +133,7 @@ PyObject* quant_cache(PyObject*, PyObject* const* a, Py_ssize_t n) {
     auto *kcp = (int8_t*)kc.data_ptr(), *vcp = (int8_t*)vc.data_ptr();
     auto* sp = (const int64_t*)slots.data_ptr();
     auto *ksp = (const float*)ks.data_ptr(), *vsp = (const float*)vs.data_ptr(), *mup = (const float*)mu.data_ptr();
-    return launch([&] {
+    return launch("kvq_quant_cache", [&] {
       return p_quant_cache(kp, key.stride(0), key.stride(1), vp, value.stride(0), value.stride(1), kcp, kc.stride(0),
                            kc.stride(1), kc.stride(2), vcp, vc.stride(0), vc.stride(1), vc.stride(2), sp, T, H, D,
                            kc.size(0), kc.size(1), ksp, kcols, vsp, vcols, mup, st);
@@ -186,8 +190,9 @@ PyObject* decode_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     auto *kp = (const int8_t*)kc.data_ptr(), *vp = (const int8_t*)vc.data_ptr();
     auto *cup = (const int32_t*)cu.data_ptr(), *slp = (const int32_t*)sl.data_ptr(), *btp = (const int32_t*)bt.data_ptr();
     auto *ksp = (const float*)ks.data_ptr(), *vsp = (const float*)vs.data_ptr();
-    return launch([&] {
-      if (group != D || rows < T)   // tokens past the buffers' rows are never cut
+    const bool ex = group != D || rows < T;   // tokens past the buffers' rows are never cut
+    return launch(ex ? "kvq_int8_decode_attention_ex" : "kvq_int8_decode_attention", [&] {
+      if (ex)
         return p_decode_ex(qp, q.stride(0), q.stride(1), kp, kc.stride(0), kc.stride(1), kc.stride(2), vp, vc.stride(0),
                            vc.stride(1), vc.stride(2), kc.size(0), bs, Hkv, D, op, out.stride(0), out.stride(1), cup, slp,
                            btp, bt.stride(0), B, Hq, ksp, kcols, vsp, vcols, scale, sop, smp, ssp, seg_st, seg_sh, S, rows,
@@ -251,7 +256,7 @@ PyObject* long_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     auto *ksp = (const float*)ks.data_ptr(), *vsp = (const float*)vs.data_ptr();
     auto *rp = (const int32_t*)treq->data_ptr(), *wp = (const int32_t*)trow->data_ptr();
     if (mode) {
-      return launch([&] {
+      return launch(pp ? "kvq_int8_prefill_attention_ex" : "kvq_int8_prefill_attention", [&] {
         return p_prefill_i8(qp, q.stride(0), q.stride(1), kp, kc.stride(0), kc.stride(1), kc.stride(2), vp, vc.stride(0),
                             vc.stride(1), vc.stride(2), nb, bs, H, D, op, out.stride(0), out.stride(1), cup, slp, btp,
                             bt.stride(0), Hq, rp, wp, tiles, rows, scale, ksp, kcols, vsp, vcols, mode == 2, pp, sp, mp, nm,
@@ -267,16 +272,20 @@ PyObject* long_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const at::Tensor kt = at::empty({P, bs, H, D}, q.options()), vt = at::empty({P, bs, H, D}, q.options());
     void *ktp = kt.data_ptr(), *vtp = vt.data_ptr();
     auto *rqp = (const int32_t*)sreq->data_ptr(), *jp = (const int32_t*)sj->data_ptr(), *tbp = (const int32_t*)tbt->data_ptr();
-    return launch([&] {
+    return launch("kvq_dequant_pages", [&] {
       const int rc = p_dequant(kp, kc.stride(0), kc.stride(1), kc.stride(2), vp, vc.stride(0), vc.stride(1), vc.stride(2), nb,
                                bs, H, D, ktp, vtp, btp, bt.stride(0), rqp, jp, P, ksp, kcols, vsp, vcols, st);
       if (rc) return rc;
+      entry = pp ? "kvq_paged_prefill_attention_ex" : "kvq_paged_prefill_attention";
       return p_prefill(qp, q.stride(0), q.stride(1), ktp, bs * H * D, H * D, D, vtp, bs * H * D, H * D, D, P, bs, H, D, op,
                        out.stride(0), out.stride(1), cup, slp, tbp, tbt->stride(0), Hq, rp, wp, tiles, rows, scale, pp, sp, mp,
                        nm, pop, pmp, st);
     });
   });
 }
+
+// (): the entry point of this thread's last call, as the Python path names it in its error
+PyObject* last_entry(PyObject*, PyObject*) { return PyUnicode_FromString(entry); }
 
 // ({name: address}): the library's entry points
 PyObject* bind(PyObject*, PyObject* d) {
@@ -301,6 +310,7 @@ PyMethodDef methods[] = {
      "kvq_int8_decode_attention on torch tensors"},
     {"long_attention", (PyCFunction)(void (*)(void))long_attention, METH_FASTCALL,
      "the long requests' attention on torch tensors"},
+    {"last_entry", last_entry, METH_NOARGS, "the entry point of this thread's last call"},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_torch_calls", "kvq operators on torch tensors", -1, methods, nullptr, nullptr,

@@ -312,7 +312,7 @@ def _served(e, op, *args):
         return False
     rc = getattr(calls, op)(*args)
     if rc == _native.ERR_LAUNCH:
-        raise _native.error(op)
+        raise _native.error(calls.last_entry())
     return rc == 0
 
 

@@ -1,13 +1,14 @@
 """kvq._torch_calls against the Python path it stands for: the same results where both serve a call, and the same
 error where the Python path refuses one."""
+import ctypes
 import threading
 
 import pytest
 import torch
 from conftest import nan_like, nan_segm
 
+from kvq import _native, synth
 from kvq import cuda_kernels as ck
-from kvq import synth
 from test_gpu_kernels import dev, int8_cache
 
 pytestmark = pytest.mark.gpu
@@ -161,3 +162,45 @@ def test_streams_and_threads():
     assert not errors
     for i in range(3):
         assert (got[i].float() - want.float()).abs().max() < 2e-2
+
+
+@pytest.mark.parametrize("failing", ["kvq_quant_cache", "kvq_int8_decode_attention", "kvq_int8_decode_attention_ex",
+                                     "kvq_dequant_pages", "kvq_paged_prefill_attention", "kvq_paged_prefill_attention_ex",
+                                     "kvq_int8_prefill_attention", "kvq_int8_prefill_attention_ex"])
+def test_launch_errors_name_the_entry_point(failing, monkeypatch):
+    """A launch the HIP runtime refuses raises what the Python path raises: entry points that return
+    KVQ_ERR_LAUNCH without launching stand in for the library's, in the native module and in ctypes."""
+    d = _case()
+    refuse, accept = (ctypes.CFUNCTYPE(ctypes.c_int)(lambda rc=rc: rc) for rc in (_native.ERR_LAUNCH, 0))
+    # (uncut work lists go to the _ex entry points too, without their lists)
+    refused = {failing, failing.replace("_attention", "_attention_ex") if "prefill" in failing else failing}
+    lib = _native.load()
+    real = {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _native.SIGNATURES}
+    stubs = {name: refuse if name in refused else accept for name in real}
+    if "decode" in failing:    # fewer rows than tokens, or one each
+        d["segm"] = nan_segm(3 if failing.endswith("_ex") else d["q"].shape[0], HQ, 4, D)
+    if "prefill" in failing or "dequant" in failing:
+        monkeypatch.setenv("KVQ_PREFILL_DIRECT", "1" if "int8" in failing else "0")
+        # cut or whole: where the estimate of a merge is small or large
+        cut = failing.endswith("_ex")
+        monkeypatch.setattr(ck, "_prefill_us", lambda longest, groups, partials, *a: (partials is None) == cut)
+
+    class Lib:
+        kvq_last_error = staticmethod(lambda: b"no such luck")
+        kvq_prefill_rows_per_tile, kvq_prefill_max_parts = lib.kvq_prefill_rows_per_tile, lib.kvq_prefill_max_parts
+
+        def __getattr__(self, name):
+            return lambda *a: _native.ERR_LAUNCH if name == failing else 0
+
+    f = _write if failing == "kvq_quant_cache" else _attend
+    ck.ext()
+    try:
+        ck.ext().calls.bind({name: ctypes.cast(s, ctypes.c_void_p).value for name, s in stubs.items()})
+        monkeypatch.setattr(_native, "_LIB", Lib())
+        native = _outcome(f, d)
+        monkeypatch.setattr(ck.ext(), "calls", None)
+        python = _outcome(f, d)
+    finally:
+        monkeypatch.undo()
+        ck.ext().calls.bind(real)
+    assert native == python == (_native.NativeError, f"{failing}: no such luck")

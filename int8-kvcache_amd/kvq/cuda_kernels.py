@@ -664,16 +664,16 @@ def long_attention(q, k_cache, v_cache, out, cu_seqlens_q, seq_lens, block_table
     _check(bs == plan.block_size, f"block size {bs} != plan block size {plan.block_size}")
     e = ext()
     work = plan.work(q.shape[1] // h, h, d, q.device)
-    if os.environ.get("KVQ_DEBUG_DUMP"):  # the prefill call's metadata, for an offline replay (kvq.debug_dump)
-        from . import debug_dump
-        debug_dump.dump_long_call(os.environ["KVQ_DEBUG_DUMP"], q, out, cu_seqlens_q, seq_lens, plan,
-                                  (plan.src_req.shape[0], bs, h, d), *plan.tiles(q.shape[1] // h, q.device),
-                                  max_query_len, e.prefill_rows, softmax_scale)
     direct = os.environ.get("KVQ_PREFILL_DIRECT")
     if direct is None:
         direct = "1" if work.direct and _direct_takes(k_cache) and _direct_takes(v_cache) else "0"
     _check(direct in ("0", "1", "fold"), f"KVQ_PREFILL_DIRECT must be 0, 1 or fold, got {direct!r}")
     ks, vs = static["k_scale"], static["v_scale"]
+    if os.environ.get("KVQ_DEBUG_DUMP"):  # the prefill call's metadata, for an offline replay (kvq.debug_dump)
+        from . import debug_dump
+        debug_dump.dump_long_call(os.environ["KVQ_DEBUG_DUMP"], q, out, cu_seqlens_q, seq_lens, plan,
+                                  (plan.src_req.shape[0], bs, h, d), work.tile_req, work.tile_row, max_query_len,
+                                  e.prefill_rows, softmax_scale, work, direct, (k_cache, v_cache, block_table, ks, vs))
     src = plan.gpu(q.device) if direct == "0" else (None, None, None)
     if _served(e, "long_attention", q, k_cache, v_cache, out, cu_seqlens_q, seq_lens, block_table, ks, vs, softmax_scale,
                ("0", "1", "fold").index(direct), e.prefill_rows, work.tile_req, work.tile_row, work.tile_piece,

@@ -7,7 +7,8 @@ describes, filled by the oracle's page dequantization -- reproduces implementati
 cache for every row the work list covers. Corrupted dumps (a table entry past the temporary cache, a key
 count past the copied pages, a work entry past a request's rows, pages of another request) are reported.
 On the GPU: the dump written by a real paged_attention call, replayed on the HIP prefill kernel, against
-the oracle on the replay's tensors.
+the oracle on the replay's tensors. Both with rows whole and cut into pieces, from the temporary cache and from the
+INT8 pages.
 """
 import os
 
@@ -98,6 +99,103 @@ def test_check_reports_corrupted_dumps(tmp_path, fault):
     assert errs and all(f"req {r}" in e for e in errs), errs
 
 
+def _cut(monkeypatch, on=True):
+    """Cut every row that can be (or none), whatever it is estimated to cost."""
+    monkeypatch.setattr(ck, "_prefill_us", lambda longest, groups, partials, *a: (partials is None) == on)
+
+
+def _dump_call(tmp_path, monkeypatch, source):
+    """The dump of a long_attention call whose rows are cut, with the kernels left out."""
+    class Nothing:
+        calls, prefill_rows, prefill_max_parts = None, ROWS, 64
+
+        def __getattr__(self, name):
+            return lambda *a: None
+
+    c, kq, vq = _batch()
+    path = str(tmp_path / "cut.pt")
+    monkeypatch.setattr(ck, "_EXT", Nothing())
+    monkeypatch.setenv("KVQ_DEBUG_DUMP", path)
+    monkeypatch.setenv("KVQ_PREFILL_DIRECT", source)
+    _cut(monkeypatch)
+    plan = ck.plan_long(c["cu"], c["seq_lens"], 16)
+    ck.long_attention(c["q"], kq, vq, torch.empty_like(c["q"]), c["cu"], c["seq_lens"], c["block_table"], 200, plan,
+                      c["scale"], c["static"])
+    return debug_dump.load(path), plan.work(7, 4, 128, torch.device("cpu"))
+
+
+@pytest.mark.parametrize("source", ["0", "1", "fold"])
+def test_dump_holds_the_list_that_runs(tmp_path, monkeypatch, source):
+    d, work = _dump_call(tmp_path, monkeypatch, source)
+    assert debug_dump.check(d) == [] and d["source"] == source and d["slots"] == work.slots > 0
+    for k in ("tile_req", "tile_row", "tile_piece", "tile_slot", "merge"):
+        assert torch.equal(d[k], getattr(work, k)), k
+
+
+@pytest.mark.parametrize("fault", ["slot_past_buffers", "slot_twice", "piece_of_none", "piece_missing", "merged_short",
+                                   "merged_twice", "not_merged", "foreign_merge", "too_many_pieces"])
+def test_check_reports_bad_pieces(tmp_path, monkeypatch, fault):
+    d, _ = _dump_call(tmp_path, monkeypatch, "0")
+    parts = d["tile_piece"] >> 16
+    i = int((parts > 2).nonzero()[0])
+    r, r0 = int(d["tile_req"][i]), int(d["tile_row"][i])
+    m = int(((d["merge"][:, 0] == r) & (d["merge"][:, 1] == r0)).nonzero()[0])
+    other = int((d["tile_slot"] != d["tile_slot"][i]).logical_and(parts > 1).nonzero()[0])
+    if fault == "slot_past_buffers":
+        d["tile_slot"][i] = d["slots"]
+    elif fault == "slot_twice":
+        d["tile_slot"][i] = d["tile_slot"][other]
+    elif fault == "piece_of_none":
+        d["tile_piece"][i] = int(parts[i]) << 16 | int(parts[i])
+    elif fault == "piece_missing":
+        for k in ("tile_req", "tile_row", "tile_piece", "tile_slot"):
+            d[k] = torch.cat([d[k][:i], d[k][i + 1:]])
+    elif fault == "merged_short":
+        d["merge"][m, 3] -= 1
+    elif fault == "merged_twice":
+        d["merge"] = torch.cat([d["merge"], d["merge"][m:m + 1]])
+    elif fault == "not_merged":
+        d["merge"] = torch.cat([d["merge"][:m], d["merge"][m + 1:]])
+    elif fault == "foreign_merge":
+        d["merge"][m, 1] += ROWS * 1000
+    else:
+        same = (d["tile_req"] == r) & (d["tile_row"] == r0)
+        d["tile_piece"][same] = (d["tile_piece"][same] & 0xffff) | 65 << 16
+    errs = debug_dump.check(d)
+    assert errs and any(f"req {r}" in e for e in errs), errs
+
+
+@pytest.mark.parametrize("source", ["0", "1"])
+@pytest.mark.parametrize("page", [-1, 10 ** 6])
+def test_check_reports_pages_outside_the_int8_cache(tmp_path, monkeypatch, source, page):
+    """Both sources start from the requests' own table: the direct kernel's pages, and the pages copied."""
+    d, _ = _dump_call(tmp_path, monkeypatch, source)
+    d["cache_table"][3, 5] = page
+    errs = debug_dump.check(d)
+    assert errs and all("req 3" in e for e in errs), errs
+
+
+def test_older_dumps_are_checked_as_whole_rows(tmp_path):
+    c, kq, vq = _batch()
+    path, *_ = _dump(tmp_path, c, kq, vq)
+    d = {k: v for k, v in debug_dump.load(path).items() if k != "source"}
+    assert "tile_piece" not in d and debug_dump.check(d) == []
+
+
+@pytest.mark.parametrize("interleaved", [True, False])
+def test_replayed_caches_keep_shape_strides_and_storage(interleaved):
+    kv = torch.zeros(6, 2, 16, 2 * 64, dtype=torch.int8)
+    by_slot = kv.permute(0, 2, 1, 3)
+    k, v = (by_slot[..., 64:], by_slot[..., :64]) if interleaved else (torch.zeros(6, 16, 2, 64, dtype=torch.int8),) * 2
+    d = {"cache_shape": tuple(k.shape), "k_stride": k.stride(), "v_stride": v.stride(), "v_offset": -64 if interleaved else None}
+    a, b = debug_dump._random_caches(d, torch.Generator().manual_seed(0), "cpu")
+    assert a.shape == b.shape == k.shape and a.stride() == k.stride() and b.stride() == v.stride()
+    assert (a.untyped_storage().data_ptr() == b.untyped_storage().data_ptr()) == interleaved
+    assert int(a.min()) == int(b.min()) == -127 and int(a.max()) == int(b.max()) == 127
+    if interleaved:
+        assert b.data_ptr() + 64 == a.data_ptr()
+
+
 @pytest.mark.gpu
 def test_dump_of_a_real_call_replays_on_the_gpu(tmp_path, monkeypatch):
     """KVQ_DEBUG_DUMP set around a mixed-batch paged_attention call: the dump is written, its bounds report
@@ -122,5 +220,46 @@ def test_dump_of_a_real_call_replays_on_the_gpu(tmp_path, monkeypatch):
     cov = ~torch.isnan(ref[:, 0, 0])
     e = O.compare(ref[cov], out.cpu()[cov])
     record("debug_dump_gpu_replay", **e)
+    assert e["rel_l2"] < 1e-2 and e["max_abs"] <= 2e-2, e
+    assert torch.isnan(out.cpu()[~cov].float()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cut", [True, False])
+@pytest.mark.parametrize("source", ["0", "1", "fold"])
+@pytest.mark.parametrize("interleaved", [True, False])
+def test_every_form_replays_as_it_ran(tmp_path, monkeypatch, cut, source, interleaved):
+    """The dumps of real calls in every form the long path takes: the list on the device is the dump's, its report
+    is clean, and the replay -- pieces merged, INT8 pages read where the call read them -- matches the oracle."""
+    c, kq, vq = _batch()
+    path = str(tmp_path / "call.pt")
+    monkeypatch.setenv("KVQ_DEBUG_DUMP", path)
+    monkeypatch.setenv("KVQ_PREFILL_DIRECT", source)
+    _cut(monkeypatch, cut)
+    if interleaved:
+        kq, vq = torch.cat([kq.cuda(), vq.cuda()], -1).split(128, -1)
+    plan = ck.plan_long(c["cu"], c["seq_lens"], 16)
+    dc = {k: (v.cuda() if isinstance(v, torch.Tensor) else v) for k, v in c.items()}
+    ck.long_attention(dc["q"], kq.cuda(), vq.cuda(), torch.empty_like(dc["q"]), dc["cu"], dc["seq_lens"], dc["block_table"],
+                      200, plan, c["scale"], {k: v.cuda() for k, v in c["static"].items()})
+    d = debug_dump.load(path)
+    assert debug_dump.check(d) == [] and ("tile_piece" in d) == cut and d["source"] == source
+    ran = {}
+    for name in ("int8_prefill_attention", "paged_prefill_attention"):
+        def run(*a, real=getattr(ck.ext(), name), name=name):
+            ran[name] = a
+            return real(*a)
+        monkeypatch.setattr(ck.ext(), name, run)
+    q, kt, vt, out = debug_dump.replay(d, seed=3)
+    torch.cuda.synchronize()
+    assert list(ran) == ["paged_prefill_attention" if source == "0" else "int8_prefill_attention"]
+    if source != "0":
+        _, k, v, *rest = ran["int8_prefill_attention"]
+        assert k.stride() == d["k_stride"] == tuple(kq.stride()) and v.stride() == d["v_stride"] == tuple(vq.stride())
+        assert rest[-2] == (source == "fold")
+    ref = oracle_replay(d, q, kt, vt)
+    cov = ~torch.isnan(ref[:, 0, 0])
+    e = O.compare(ref[cov], out.cpu()[cov])
+    record("debug_dump_forms", cut=cut, source=source, **e)
     assert e["rel_l2"] < 1e-2 and e["max_abs"] <= 2e-2, e
     assert torch.isnan(out.cpu()[~cov].float()).all()

@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the static INT8 KV-cache hot path on one MI355X.
 
-Headline (BASELINE.json metric, config c2): INT8 paged decode attention, 128 requests x 32768 keys,
+Headline (config c2): INT8 paged decode attention, 128 requests x 32768 keys,
 28 q / 4 kv heads, head_dim 128, block 16, in vLLM's interleaved [nb, H, bs, 2D] int8 cache (filled
 with c0-distribution codes by this package's quantize-and-cache kernel), shuffled block tables over
 263,168 blocks. A step is one kvq.cuda_kernels.decode_attention call made as the vLLM backend makes it
@@ -37,8 +37,7 @@ import torch  # noqa: E402
 from kvq import _native, synth  # noqa: E402
 from kvq import cuda_kernels as ck  # noqa: E402
 
-with open(os.path.join(REPO, "BASELINE.json")) as _f:
-    METRIC = json.load(_f)["metric"]
+METRIC = "INT8 paged decode attn µs + HBM GB/s (128×32k, 28q/4kv, d128, block16)"
 PEAK_BF16_TFLOPS = 2500.0   # MI355X dense bf16 MFMA
 PEAK_GBS = 8000.0          # MI355X HBM3E
 PEAK_INT8_OPS = 5.0e15     # dense int8 MFMA
@@ -49,7 +48,7 @@ DEV = "cuda"
 class HipEvents:
     """Raw hipEvent_t pairs, for timing only: created without the system-scope fence at record
     (hipEventDisableSystemFence), whose cache writeback and invalidation cost ~2.5 us per recorded
-    event on these boxes. The library records pairs around its next attention kernel
+    event on this platform. The library records pairs around its next attention kernel
     (kvq_set_attention_events); record() puts one on a given stream."""
 
     DISABLE_SYSTEM_FENCE = 0x20000000
@@ -185,7 +184,7 @@ def read_ceiling(buf, reps=10):
 def mfma_ceiling(reps=5):
     """TFLOP/s of back-to-back dense bf16 MFMAs (the library's kvq_mfma_probe: 16x16x32, the prefill
     kernel's instruction) on random bf16 operands, 8 workgroups of 4 wavefronts per CU, ~7 ms per launch,
-    timed as the prefill kernel is (graph replays of 3 calls): the rate the box delivers under its power
+    timed as the prefill kernel is (graph replays of 3 calls): the rate the card delivers under its power
     limit over such a burst, the ceiling beside the prefill kernel's rate."""
     g = torch.Generator(device=DEV).manual_seed(11)
     data = torch.randn(8192, generator=g, device=DEV).to(torch.bfloat16)

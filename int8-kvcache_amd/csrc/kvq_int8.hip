@@ -63,7 +63,7 @@ constexpr int DEFAULT_SEG_COST_V32 = 12;  // the same for verify_kernel with one
 // register ring of the decode kernel: tiles in flight per wavefront (PF - 1 ahead of the one computed).
 // Under full load HBM latency grows with the bytes in flight (~5 us at 2 tiles ahead per wavefront), and
 // every piece of a segment pays it twice at its start (page ids, then K/V): one tile ahead streams as
-// fast and starts pieces sooner (same-box A/B: c4 decode rows 128.2 -> 124.9 us, c2 645 -> 643 us).
+// fast and starts pieces sooner (A/B on one card: c4 decode rows 128.2 -> 124.9 us, c2 645 -> 643 us).
 constexpr int DEFAULT_PREFETCH = 2;
 constexpr int DEFAULT_V32_RING = 2;     // verify_kernel's ring slots (3 with one key split)
 constexpr int DEFAULT_V32_KSPLIT = 2;   // verify_kernel's key splits per workgroup
@@ -683,7 +683,7 @@ constexpr int PLAN_CACHE = 4;
 // workers [x q + min(x, rem), ...) for active = 8 q + rem -- consecutive ranges that tile [0, active)
 // exactly. Counting the workers with units, not the grid, spreads a small batch over all 8 XCDs: an XCD
 // draws about an eighth of the HBM bandwidth, and a batch with fewer pieces than workgroups otherwise
-// filled the first XCDs only (attention + merge in a graph, same box: 1 x 4,096 keys 18.2 -> 15.0 us,
+// filled the first XCDs only (attention + merge in a graph, same card: 1 x 4,096 keys 18.2 -> 15.0 us,
 // 8 requests of about 2k 21.9 -> 18.1, 1 x 32k 48.8 -> 36.7, 4 x 8-token verification of 4k 24.5 -> 20.3;
 // full grids unchanged). KVQ_XCD_ORDER=0 makes worker = block.
 __device__ Plan plan_and_locate(const AttnArgs& a, int lane, int& worker_out, int& r_out, long long& start_out,
@@ -771,7 +771,7 @@ __device__ Plan plan_and_locate(const AttnArgs& a, int lane, int& worker_out, in
 // worker where it starts, one piece. Positions are counted from the worker's first unit, so that a piece's number
 // needs a small quotient by the chunk and only where the segment reaches beyond this worker. The front of a
 // kernel, entry to first page id, took 3.0 us with 64-bit positions and divisions, 2.4 of them arithmetic; with
-// this and fresh_args, in graphs on one box: 1 x 4,096 keys 14.9 -> 14.3 us, 8 x 2k 17.9 -> 17.3, 24 x 4-token
+// this and fresh_args, in graphs on one card: 1 x 4,096 keys 14.9 -> 14.3 us, 8 x 2k 17.9 -> 17.3, 24 x 4-token
 // verification 25.7 -> 24.0, 64 x 8 57.9 -> 56.8, c4's ragged decode rows 104.6 -> 103.4, 128 x 32k unchanged.
 template <typename F>
 __device__ __forceinline__ void walk_pieces(const AttnArgs& a, int lane, F&& f) {
@@ -879,7 +879,7 @@ __device__ __forceinline__ void transpose4x4(uint32_t a0, uint32_t a1, uint32_t 
 constexpr int MERGE_FIELDS = 36;  // 32 accumulators (D = 128), max, denominator, 2 spare
 constexpr int MERGE_SLOTS = MAX_ROW_TILES - 1;
 // Up to this many (request, kv head) pairs a decode workgroup holds 4 key splits instead of 2: few pieces, so more
-// wavefronts on each (same box, 2 and 4: 1 x 32k 35.8 and 28.6 us, 4 x 14k 26.0 and 24.1, 16 x 3k of 14 / 2 heads d64
+// wavefronts on each (same card, 2 and 4: 1 x 32k 35.8 and 28.6 us, 4 x 14k 26.0 and 24.1, 16 x 3k of 14 / 2 heads d64
 // 14.6 and 13.8, 16 x 2k 18.5 and 18.1, 8 x 2k 15.9 and 15.8; 12 x 4k of 32 / 8 heads, 96 pairs, 23.5 and 23.9; 48 ragged
 // of 32 / 8, 384 pairs, 34.8 and 37.1).
 constexpr int WIDE_SPLIT_PAIRS = 64;
@@ -943,7 +943,7 @@ __device__ __forceinline__ void attend_segment(int seq, int tok, int qlen, int s
   const AttnArgs& a = fresh_args();
   const bool active = row0 < qlen * a.G;
   // what the tile loop reads, held in registers (a field read in the loop was loaded again every tile: one-pass 64 x 8
-  // verification 155.3 -> 150.5 us, 24 x 4 87.2 -> 84.5; 1 x 4,096 decode 13.7 -> 13.5, same box)
+  // verification 155.3 -> 150.5 us, 24 x 4 87.2 -> 84.5; 1 x 4,096 decode 13.7 -> 13.5, same card)
   const int num_blocks = a.num_blocks, lbs = a.lbs;
   const int64_t k_sb = a.k_sb, k_sn = a.k_sn, v_sb = a.v_sb, v_sn = a.v_sn;
   constexpr int KPL = D / 4;        // K bytes per lane and key
@@ -1327,7 +1327,7 @@ __device__ __forceinline__ int swz_v(int row) { return ((((row >> 1) & 1) | (((r
 // dot is scaled by that group's q scale and the groups' scores are summed in fp32.
 // Wave priority over the issue of a step's tile DMA (after the step's barrier): the wavefront puts its
 // share of the next tile's requests out ahead of the SIMD's other wavefronts' tile arithmetic, so the
-// ring's loads start sooner (c3 60.1 -> 59.4 us, same box; priority over the QK block as well: no
+// ring's loads start sooner (c3 60.1 -> 59.4 us, same card; priority over the QK block as well: no
 // change). 0: off.
 constexpr int V32_DMA_PRIO = 1;
 template <int P>
@@ -1345,7 +1345,7 @@ __device__ __forceinline__ void attend_rows32(int seq, int tok, int qlen, int se
   const AttnArgs& a = fresh_args();
   const bool active = row0 < qlen * a.G;
   // what the tile loop reads, held in registers (a field read in the loop was loaded again every tile: one-pass 64 x 8
-  // verification 155.3 -> 150.5 us, 24 x 4 87.2 -> 84.5; 1 x 4,096 decode 13.7 -> 13.5, same box)
+  // verification 155.3 -> 150.5 us, 24 x 4 87.2 -> 84.5; 1 x 4,096 decode 13.7 -> 13.5, same card)
   const int num_blocks = a.num_blocks, lbs = a.lbs;
   const int64_t k_sb = a.k_sb, k_sn = a.k_sn, v_sb = a.v_sb, v_sn = a.v_sn;
   constexpr int KST = D / 32;       // 32-channel QK steps = 32-channel PV tiles
@@ -1847,7 +1847,7 @@ __global__ __launch_bounds__(WAVE * 2 * KS) void verify_kernel(AttnArgs a) {
 // merge needs neither the plan nor any buffer beyond the split buffers of the call.
 constexpr int RED_WAVES = 4;
 constexpr int MERGE_Z = 64;   // largest z extent of split_reduce_kernel's grid
-// pieces of a row fetched together with its denominators (c3: 59.4 -> 59.0 us same box, c4 unchanged;
+// pieces of a row fetched together with its denominators (c3: 59.4 -> 59.0 us same card, c4 unchanged;
 // 4 pieces: 61.4 us -- the extra reads of rows with fewer pieces cost more than the round trip saves)
 constexpr int MERGE_SPEC = 2;
 template <int D>
@@ -1856,7 +1856,7 @@ __device__ __forceinline__ void merge_row(const AttnArgs& a, int tok, int t, int
   // otherwise pieces 0..S-2 hold l >= 0 and the last piece -2 - l
   const int64_t base = (int64_t)(tok + t) * a.seg_st + (int64_t)h * a.seg_sh;
   // the maxima and the first MERGE_SPEC pieces' partial outputs are fetched with the denominators (one
-  // memory round trip for a row of up to MERGE_SPEC pieces), later pieces four at a time
+  // memory round trip for a row of up to MERGE_SPEC pieces), later pieces 8 at a time while more than 4 are left, else 4
   const bool held = lane < a.max_splits;
   constexpr int CPL = D / WAVE;
   const float* po = a.segm_out + base * D + CPL * lane;
@@ -1912,7 +1912,7 @@ __device__ __forceinline__ void merge_row(const AttnArgs& a, int tok, int t, int
       for (int e = 0; e < CPL; ++e) num[e] = in ? __builtin_fmaf(ws, v[j][e], num[e]) : num[e];
     }
   };
-  // a row of many pieces (a small batch's) reads 8 at a time, one of few 4: in graphs, same box, 4 / 8 / 14 at a time
+  // a row of many pieces (a small batch's) reads 8 at a time, one of few 4: in graphs, same card, 4 / 8 / 14 at a time
   // 8 x 2k keys 15.8 / 15.5 / 15.3 us, 1 x 4,096 14.7 / 14.5 / 14.4, c4's decode rows 99.2 / 98.8 / 98.8, 64 x 8-token
   // verification (few pieces a row) 56.1 / 55.8 / 56.6
   int s0 = MERGE_SPEC;
@@ -1993,7 +1993,7 @@ __device__ __forceinline__ u32x4 dq8x(uint32_t w0, uint32_t w1, const float (&s)
 // (16 lanes per 256-byte K or V row at D = 128), never parts of lines.
 constexpr int DQ_BATCH = 16;
 // Few pages leave CUs idle and their workgroups a serial run of tokens, so a page's tokens are split over grid.z
-// down to DQ_MIN_TOKENS, up to about DQ_WG_PER_CU workgroups per CU (whole prefill calls in a graph, same box: 479
+// down to DQ_MIN_TOKENS, up to about DQ_WG_PER_CU workgroups per CU (whole prefill calls in a graph, same card: 479
 // tokens of 498, 32 / 8 heads, blocks of 64 slots 30.4 -> 22.7 us, 157 of 157, 16 / 16 heads d64 19.8 -> 11.7, 1,024 of
 // 1,024 in blocks of 32 34.6 -> 33.3; 512 pages of 16 slots unchanged; slices of 16 tokens 23.8 and 12.7).
 constexpr int DQ_WG_PER_CU = 4, DQ_MIN_TOKENS = 4;
@@ -2115,7 +2115,7 @@ constexpr int PR_STAGES = 3;                // LDS ring: tiles in flight + the o
 constexpr int PR_I8_STAGES = 2;             // INT8 pages: int8 ring stages (2 x 8 KB at D 128, + 2 bf16 stages)
 // Wave priority over a tile's QK block (K operand reads + MFMAs): a wavefront with matrix work ready
 // issues it ahead of the other wavefronts' softmax VALU on its SIMD, so the MFMA pipe idles less
-// (c4 prefill 7.28-7.37 -> 7.16-7.19 ms, same box, identical output; priority over the PV block as well,
+// (c4 prefill 7.28-7.37 -> 7.16-7.19 ms, same card, identical output; priority over the PV block as well,
 // or over the PV block alone, timed the same or slower, and over the softmax made no difference).
 // 0: off.
 constexpr int PR_QK_PRIO = 1;
@@ -2916,7 +2916,7 @@ __global__ __launch_bounds__(WAVE * PR_MERGE_WAVES) void prefill_merge_kernel(Pr
 // independent accumulation chains of v_mfma_f32_16x16x32_bf16 (the prefill kernel's instruction) for
 // `iters` rounds, on operands taken from `data` (1,024 16-byte vectors) and rotated every round, so the
 // multipliers see changing values as the prefill's do; each lane stores a sum of its accumulators (no
-// MFMA is dropped). What it sustains is the dense bf16 rate the box delivers, at the clock its power
+// MFMA is dropped). What it sustains is the dense bf16 rate the card delivers, at the clock its power
 // limit allows for such operands: the ceiling the prefill kernel is compared with.
 __global__ __launch_bounds__(256) void mfma_probe_kernel(const bf16x8* __restrict__ data, int iters,
                                                          float* __restrict__ out) {
@@ -2947,7 +2947,7 @@ __global__ __launch_bounds__(256) void mfma_probe_kernel(const bf16x8* __restric
 // once and stores each lane's XOR of what it read (so no load is dropped). Workgroup b streams the
 // b-th contiguous share of the buffer, its wavefronts taking interleaved 1 KB blocks of it with 8
 // non-temporal loads in flight per lane -- the way the attention kernel streams its pages. What it
-// sustains is what HBM delivers to a read-only stream on the box at hand: the ceiling the decode
+// sustains is what HBM delivers to a read-only stream on the card at hand: the ceiling the decode
 // attention kernel is compared with.
 // ------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void stream_read_kernel(const u32x4* __restrict__ p, int64_t n16,
@@ -2978,7 +2978,7 @@ __global__ __launch_bounds__(256) void stream_read_kernel(const u32x4* __restric
 // two streams interleaved in the fixed ratio KR : KW (per round a lane reads KR chunks and writes KW,
 // each value a function of what it read). Timed at a kernel's byte mix -- 2 : 1 for the fused cache
 // write (bf16 K/V read, int8 codes written), 1 : 2 for page dequantization (int8 read, bf16 written) --
-// it gives what a plain stream of that many bytes costs on the box, the floor that kernel is compared
+// it gives what a plain stream of that many bytes costs on the card, the floor that kernel is compared
 // with.
 template <int KR, int KW>
 __global__ __launch_bounds__(256) void stream_rw_kernel(const u32x4* __restrict__ src, int64_t nr,
@@ -3110,7 +3110,7 @@ int seg_cost_units(const Tuning& t, int v32_key_splits) {
   // verify_kernel with 2 key splits streams a unit (one 32-key tile of the segment) in half the time, so
   // its fixed cost is more units (c3, 3-slot rings: 12 -> 24 units 68.5 -> 66.1 us, 36 units 67.3, 48
   // units 71.3; 2-slot rings: 16 units 65.1-65.3 us, 24 units 66.1-66.9; with the merge's speculative
-  // loads, same box: 10, 12, 14, 16, 20 units 59.7, 59.3, 58.6, 59.0, 60.3 us -- a piece's measured fixed
+  // loads, same card: 10, 12, 14, 16, 20 units 59.7, 59.3, 58.6, 59.0, 60.3 us -- a piece's measured fixed
   // cost, prologue + epilogue + the step between pieces, is ~6.5 us, about 10 tiles at 1.35 us per step of
   // 2 tiles; a little more than that balances best, as the plan's first piece of a worker also waits for
   // the plan)

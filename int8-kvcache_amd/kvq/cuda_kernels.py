@@ -11,8 +11,9 @@ raises if it is missing -- there is no fallback.
 Attention on the INT8 cache is split by query length (reference kvq/cuda_kernels.py:1-11):
   * requests with at most SHORT_Q query tokens run the INT8 MFMA kernel (implementation B);
   * longer ones have their pages dequantized into a bf16 paged cache (dequant_pages, HIP) that a
-    bf16 prefill attention reads (implementation A). The page table of that temporary cache comes
-    from plan_long(), once per step for all layers.
+    bf16 prefill attention reads (implementation A), or, where that is faster (few rows per key),
+    one kernel reads the INT8 pages itself with the same output bits. The page table of the temporary
+    cache comes from plan_long(), once per step for all layers.
 In a mixed batch the long requests run first, then the INT8 kernel writes the short requests' rows.
 
 Everything is enqueued on the current torch stream; no call synchronises the host except the
@@ -198,7 +199,7 @@ class _Ext:
                      ks.data_ptr(), kcols, vs.data_ptr(), vcols, _stream(kc))
 
     # consumer of the temporary cache: in place of flash_attn_varlen_func (kvq/cuda_kernels.py:128-130)
-    # (split = LongPlan.pieces' list in place of the whole rows' tile_req / tile_row, with its buffers)
+    # (split = PrefillWork.split's lists and buffers, where tile_req / tile_row list pieces of rows)
     def paged_prefill_attention(self, q, kt, vt, out, cu_q, seq_lens, block_table, tile_req, tile_row, softmax_scale,
                                 split=None):
         n = tile_req.shape[0]
@@ -321,7 +322,8 @@ def quant_q(q, k_scale, group=None):
     return tuple(ext().quant_q(q, k_scale, group or q.shape[-1]))
 
 
-MIN_SPLIT_KEYS = 128   # the kernels never cut a split shorter than 4 tiles of 32 keys
+MIN_SPLIT_KEYS = 128   # 4 tiles of 32 keys, the shortest share of a batch a worker is given (what is left of a
+                       # segment in it may be shorter)
 
 
 def choose_splits(max_context):

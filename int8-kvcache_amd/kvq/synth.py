@@ -1,6 +1,6 @@
-"""Seeded synthetic workloads of the benchmark configurations (BASELINE configs c0..c4).
+"""Seeded synthetic workloads of the benchmark configurations (c0..c4).
 
-Host-side generators draw with numpy PCG64, so the CPU container and the GPU box produce identical
+Host-side generators draw with numpy PCG64, so a machine without a GPU and one with it produce identical
 inputs for the same seed. The multi-GB caches of the large configurations are filled on the GPU
 instead (torch generator + this package's quantize-and-cache kernel).
 

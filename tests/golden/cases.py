@@ -1,7 +1,7 @@
 """Definitions of the seeded parity cases shared by the golden-vector script and the tests.
 
 Inputs are regenerated from numpy PCG64 seeds (kvq/synth.py), so the fixtures hold only outputs and
-checksums. Shapes follow the reference's test cases (tests/conftest.py:69-88) and BASELINE config c0.
+checksums. Shapes follow the reference's test cases (tests/conftest.py:69-88) and config c0.
 """
 import importlib.util
 import os
@@ -29,7 +29,7 @@ def build(name):
         c = synth.c0_case(per_channel=name == "c0_pc")
         c["per_channel"] = name == "c0_pc"
     elif name == "c0_pc_nomu":
-        # config c0 as BASELINE.json states it: static per-channel scales, k_mu = 0 (no smooth-K)
+        # config c0: static per-channel scales, k_mu = 0 (no smooth-K)
         c = synth.c0_case(per_channel=True, smooth=False)
         c["per_channel"] = True
     elif name in ("short_28_4", "short_14_2_d64", "short_32_8_ph"):

@@ -1,6 +1,6 @@
 """Writes tests/golden/golden.safetensors + golden.json from the REFERENCE's own Python numerics.
 
-Run in the build container only (the reference is not on the GPU box and never leaves it):
+Run where the reference's sources are (/root/reference):
     python tests/golden/make_golden.py [/root/reference]
 It imports the reference's kvq.quant, kvq.ref_attn and kvq.int8_ref (pure PyTorch, CPU) to produce,
 for each case of tests/golden/cases.py:

@@ -1,5 +1,5 @@
 """HIP-graph capture (the reference's tests/test_cudagraph.py) and parity at the benchmark sizes
-(configs c2, c3, c4 of BASELINE.json), through size-independent checks: sampled requests against the
+(configs c2, c3, c4), through size-independent checks: sampled requests against the
 CPU oracle, split-count invariance, and the bit-exact cache codes of the GPU fill."""
 import math
 import os

@@ -44,7 +44,7 @@ def oracle_attention(c, kq, vq, per_channel=True, short_q=8, q_arith="fp32"):
 
 
 def check_attention(ref, out, what, ref_fp64=None, **kw):
-    """Strict bar (BASELINE): max-abs <= 2e-2, mean-abs <= 2e-3 of the bf16 kernel output against B in
+    """Strict bar: max-abs <= 2e-2, mean-abs <= 2e-3 of the bf16 kernel output against B in
     fp32 with the kernel's q contract; plus the reference's own bar (rel_l2 < 5e-3,
     tests/test_cuda_kernels.py:75) against int8_ref's fp64 q rounding when given."""
     err = O.compare(ref, out.cpu())
@@ -123,7 +123,7 @@ def test_quant_cache_head_counts_and_packed_qkv(H, D, layout, qc_kernel):
 
 
 def test_quant_cache_c1_full_size_bit_exact(qc_kernel):
-    """BASELINE config c1: 16384 tokens x 4 x 128, ~2% padded slots, 4096 x 16 interleaved cache."""
+    """Config c1: 16384 tokens x 4 x 128, ~2% padded slots, 4096 x 16 interleaved cache."""
     c = synth.c1_inputs()
     nb, bs = c["num_blocks"], c["block_size"]
     kv = torch.zeros(nb, 4, bs, 256, dtype=torch.int8)

@@ -10,7 +10,7 @@ from test_gpu_kernels import _check_dequant, _random_pages, check_attention, dev
 pytestmark = pytest.mark.gpu
 
 # key counts of the requests: from one piece of one request up to several pieces per XCD, with counts around
-# multiples of the 8 XCDs (2 kv heads, pieces of at least 8 tiles of 32 keys)
+# multiples of the 8 XCDs (2 kv heads, worker shares of at least 4 tiles of 32 keys, fixed cost included; 8 for q_len 8)
 BATCHES = {"one_tile": [1], "one_piece": [200], "three": [200, 40, 1], "eight": [256, 256, 256, 250],
            "nine": [300, 600, 33, 513], "long": [5000], "long_and_short": [7, 9000, 16, 1025]}
 

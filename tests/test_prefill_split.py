@@ -47,17 +47,20 @@ def test_split_rows_covers_every_tile_once(batch, group, hkv, d):
     for i in range(preq.shape[0]):
         count.setdefault((int(preq[i]), int(prow[i]), int(parts[i])), []).append((int(part[i]), int(slot[i])))
     assert len(count) == req.shape[0]
-    used, longest_seen = [], 0
+    used, longest_seen, shortest = [], 0, max(tiles)
     cut = {(int(a), int(b)): (int(c), int(n)) for a, b, c, n in merge}
     for (r, w, n), got_parts in count.items():
         t = int(tiles[(req == r) & (row == w)][0])
         assert sorted(p for p, _ in got_parts) == list(range(n)) and n <= min(64, t)
         longest_seen = max(longest_seen, -(-t // n))
         if n > 1:
+            shortest = min(shortest, t // n)
             first, merged = cut.pop((r, w))
             assert merged == n and all(s == first + p for p, s in got_parts)
             used += [s for _, s in got_parts]
     assert not cut and sorted(used) == list(range(slots)) and longest_seen == longest
+    # equal shares of rows longer than the length aimed at: at least half of it (rounded up)
+    assert shortest >= (ck.PREFILL_MIN_PIECE + 1) // 2
     assert preq.shape[0] * hkv <= ck.PREFILL_PER_CU * 256 and longest >= ck.PREFILL_MIN_PIECE
 
 

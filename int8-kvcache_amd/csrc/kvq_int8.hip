@@ -2272,7 +2272,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
   const char* vh = I8 ? (const char*)a.vc + (int64_t)kvh * a.v_sh : (const char*)(a.vc + (int64_t)kvh * a.v_sh);
   // Pages as one run: when the pages the workgroup reads are consecutive ids p_0, p_0 + 1, ... and a
   // page is bs slots (the layout dequant_pages writes), key k is slot p_0 bs + k of the head's cache:
-  // the tiles' addresses need no block-table read (checked once, by every wavefront alike; four table
+  // the tiles' addresses need no block-table read (within 4 GiB, run_fits; checked once, by every wavefront alike; four table
   // reads in flight per lane, over the pages of this workgroup's own tiles; the first page's id comes with
   // them, and a piece's place in the split list is read while the wavefronts meet at the end, not after: two
   // memory round trips less per workgroup, 700 + 333 tokens at up to 2,500 keys 50.6 -> 49.6 us).
@@ -2293,7 +2293,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) bad |= id[u] - pfirst != min(j0 + lane + u * WAVE, pg_hi);
     }
-    linear = !__any(bad);
+    linear = !__any(bad) && run_fits(pg_hi + 1, a.kpage) && run_fits(pg_hi + 1, a.vpage);
   }
   const char* klin = kh + (int64_t)pfirst * a.kpage;
   const char* vlin = vh + (int64_t)pfirst * a.vpage;
@@ -2312,10 +2312,10 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
     if (lin) {
       // the upper half as below: past the last page (bs == 16) it re-reads the lower half's page
       const uint32_t k1 = ((min(kb0 + 16, klast) >> a.lbs) << a.lbs) + ((kb0 + 16) & bsm);
-      kb[0] = klin + run_offset(kb0, a.krow);
-      vb[0] = vlin + run_offset(kb0, a.vrow);
-      kb[1] = klin + run_offset(k1, a.krow);
-      vb[1] = vlin + run_offset(k1, a.vrow);
+      kb[0] = klin + (uint32_t)kb0 * a.krow;
+      vb[0] = vlin + (uint32_t)kb0 * a.vrow;
+      kb[1] = klin + k1 * a.krow;
+      vb[1] = vlin + k1 * a.vrow;
     } else {
       const int i0 = kb0 >> a.lbs, i1 = min(kb0 + 16, klast) >> a.lbs;
       int p0 = __builtin_amdgcn_readfirstlane(((const __attribute__((address_space(4))) int*)bt)[i0]);

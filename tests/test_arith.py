@@ -34,9 +34,9 @@ def test_division_free_codes_match_ieee_codes(tmp_path):
     assert rc == 0 and out.endswith("mismatched 0"), out
 
 
-def test_page_run_offsets_do_not_wrap(tmp_path):
-    """prefill_body's offset of a key within a run of consecutive pages (run_offset, csrc/page_run.h): the full
-    product, also more than 4 GiB from the run's first key (524,288 keys of 32 kv heads in the bf16 cache)."""
+def test_page_runs_with_32_bit_offsets_do_not_wrap(tmp_path):
+    """The runs of consecutive pages whose keys prefill_body addresses by 32-bit offsets (run_fits, csrc/page_run.h):
+    none reaches past 4 GiB (524,288 keys of 32 kv heads in the bf16 cache), and no shorter one is left out."""
     rc, out = _run_c(tmp_path, "page_run_check")
     assert rc == 0 and out.endswith("mismatched 0"), out
 

@@ -78,3 +78,21 @@ def test_dequant_token_slices_bit_exact(D, bs, pages, H, per_channel):
     """Few pages: a page's tokens over several workgroups (slices of 4 tokens and up, a last one shorter)."""
     kq, vq, bt, src_req, src_j, st = _random_pages(max(pages, 4), bs, H, D, pages, pages + bs, per_channel)
     _check_dequant(kq, vq, bt, src_req, src_j, st)
+
+
+@pytest.mark.parametrize("requests", [16, 17])
+@pytest.mark.parametrize("q_len", [2, 3, 4, 5])
+def test_row_and_pair_counts_around_the_kernel_rule(q_len, requests):
+    """16, 24, 32 and 40 rows per kv head of 16 and 17 (request, kv head) pairs, cut and whole: one row tile, two
+    of attn_kernel or verify_kernel, as verify_rows has it, against the oracle."""
+    lens = [max(q_len, (97 * i * i + 60) % 1400) for i in range(requests)]
+    params = synth.channel_params(1, 128)
+    c = synth.paged_case(8, 1, [q_len] * requests, lens, seed=60 + q_len, params=params)
+    c["static"] = synth.calibration_scales(1, 128, params)
+    c["scale"] = 128 ** -0.5
+    kq, vq = int8_cache(c)
+    d, ref = dev(c), oracle_attention(c, kq, vq)
+    for segm in (nan_segm(d["q"].shape[0], 8, 16, 128), None):
+        out = ck.decode_attention(d["q"], dev(kq), dev(vq), nan_like(d["q"]), d["cu"], d["seq_lens"], d["block_table"],
+                                  c["scale"], d["static"], segm=segm, max_query_len=q_len)
+        check_attention(ref, out, "kernel_rule", requests=requests, q_len=q_len, segm=segm is not None)
